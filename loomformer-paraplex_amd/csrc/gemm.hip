@@ -8,7 +8,11 @@
 // K-contiguous in LDS with rows padded to 144 B, so the 16-byte fragment reads
 // of 16 consecutive rows fall in distinct banks.
 //
-// fp32/fp16: SIMT tile 64x64x16, 4x4 outputs per thread, fp32 FMA.
+// Few rows in bf16, and fp32 from 9 rows on: MFMA operands loaded straight from
+// global memory, k split over the waves of a block (gemm_frag.h).
+//
+// fp16, and fp32 with rows that are not whole 16-byte pieces: SIMT tile
+// 64x64x16, 4x4 outputs per thread, fp32 FMA.
 //
 // "Gather" mode is the grouped W_imag product of ParaplexFFN: the activation
 // row of hidden group g is the concatenation of sector slices
@@ -329,8 +333,8 @@ using BgTall = BgCfg<256, 192, 8, 4, 1, 2, 4>;
 // (the chunked prefill: 63.8 -> 62.0 ms)
 using BgTallS = BgCfg<128, 192, 4, 2, 1, 2, 4>;
 
-// Source and element offset (within the source's row) of the 32 packed
-// columns [kk, kk + 32) of group g in gather mode; they lie in one sector.
+// Source and element offset (within the source's row) of the packed columns
+// from kk on of group g in gather mode (a run of them that lies in one sector).
 __device__ __forceinline__ void gather_half(const GemmArgs& a, int64_t kk, int64_t g,
                                             const void*& src, int64_t& col) {
     const int64_t HD = a.HD, Nm = a.Nm;
@@ -917,6 +921,10 @@ gemm_bf16_big_kernel(GemmArgs a) {
         }
     }
 }
+
+}  // namespace loom
+#include "gemm_frag.h"
+namespace loom {
 
 // ------------------------------------------------------------------ skinny bf16 (M <= 64)
 // Decode-shaped products: the weight is streamed once and dominates traffic.
@@ -1604,6 +1612,94 @@ static void launch_big(const GemmArgs& a, BigTile tile, int64_t nsplit, hipStrea
     }
 }
 
+// Wave tile of a direct-fragment product (gemm_frag.h): the largest that still
+// gives 3/4 of the CUs a block and does not pad M to twice its rows.  Measured
+// over M = 32 .. 2048 at 768 x 768, 3072 x 768, 768 x 3072 and the W_imag
+// gather, that tile was the fastest or within 5% of it in both types (bf16
+// 768 x 3072: M = 64 7.0 us in 16 x 16 tiles, 128 9.2 in 32 x 16, 256 11.1 in
+// 32 x 32, 512 15.0 in 64 x 32, 999 20.9 in 64 x 64; the neighbouring sizes
+// 8.5, 10.8, 15.0, 18.7, 27.7).
+struct FragTile { int tm, tn; };
+static FragTile frag_tile(int64_t M, int64_t N, bool gather, int64_t Hq) {
+    static constexpr FragTile kTiles[] = {{64, 64}, {64, 32}, {32, 32}, {32, 16}};
+    for (const FragTile& t : kTiles)
+        if (2 * M > t.tm && (!gather || Hq % t.tn == 0) &&
+            4 * ceil_div(M, t.tm) * ceil_div(N, t.tn) >= 3 * (int64_t)device_cus())
+            return t;
+    return FragTile{16, 16};
+}
+
+// What the direct-fragment kernels need of a product: whole units of k, 16-byte
+// operands, 32-bit offsets within a tile, gather halves inside one sector and
+// n-tiles inside one q-head group.
+template <typename T, bool GATHER>
+static bool frag_fits(const GemmArgs& a) {
+    constexpr int64_t E = (int64_t)sizeof(T), V = 16 / E;
+    bool ok = a.K % kFragK<T> == 0 && a.ldw % V == 0 && ((uintptr_t)a.W & 15) == 0 &&
+              (64 * a.ldw + a.K) * E < (1LL << 31);
+    if (GATHER) {
+        ok = ok && a.HD % (64 / E) == 0 && a.Nm % (64 / E) == 0 && a.Hq % 16 == 0 && 64 * a.Nm * E < (1LL << 31);
+        for (int s = 0; s < 5; ++s) ok = ok && ((uintptr_t)a.src[s] & 15) == 0;
+    } else {
+        ok = ok && a.ldx % V == 0 && ((uintptr_t)a.X & 15) == 0 && (64 * a.ldx + a.K) * E < (1LL << 31);
+    }
+    if (a.X2 != nullptr)
+        ok = ok && a.K1 % kFragK<T> == 0 && a.ldx2 % V == 0 && a.ldw2 % V == 0 &&
+             (((uintptr_t)a.X2 | (uintptr_t)a.W2) & 15) == 0 && (64 * a.ldx2 + a.K) * E < (1LL << 31) &&
+             (64 * a.ldw2 + a.K) * E < (1LL << 31);
+    return ok;
+}
+
+template <typename T, int MT, int NT, int KW, int SP, int U, bool GATHER, bool DUAL>
+static void launch_frag_cfg(const GemmArgs& a, hipStream_t st) {
+    using C = FragCfg<T, MT, NT, KW, SP, U>;
+    const dim3 grid((unsigned)(ceil_div(a.M, C::BM) * ceil_div(a.N, C::BN)));
+    hipLaunchKernelGGL((gemm_frag_kernel<T, MT, NT, KW, SP, U, GATHER, DUAL>), grid, dim3(C::THREADS), 0, st, a);
+}
+template <typename T, bool GATHER, bool DUAL>
+static void launch_frag(const GemmArgs& a, hipStream_t st) {
+    const FragTile t = frag_tile(a.M, a.N, GATHER, a.Hq);
+    constexpr bool F32 = sizeof(T) == 4;
+    if (t.tm == 64 && t.tn == 64) {
+        // eight k parts (one block per CU) or four (two blocks per CU), whichever
+        // fills its rounds better; many fp32 tiles: 2 x 2 waves per block and no
+        // k split (4096 x 3072 x 768: 182 against 215 us)
+        const int64_t n = ceil_div(a.M, 64) * ceil_div(a.N, 64), c = device_cus();
+        if constexpr (F32 && !DUAL) {
+            if (n >= 8 * c && (!GATHER || a.Hq % 128 == 0)) return launch_frag_cfg<T, 4, 4, 1, 2, 1, GATHER, DUAL>(a, st);
+        }
+        if (n <= c || ceil_div(n, c) < 2 * ceil_div(n, 2 * c)) return launch_frag_cfg<T, 4, 4, 8, 1, 1, GATHER, DUAL>(a, st);
+        return launch_frag_cfg<T, 4, 4, 4, 1, 1, GATHER, DUAL>(a, st);
+    }
+    if (t.tm == 64) return launch_frag_cfg<T, 4, 2, F32 ? 4 : 8, 1, 1, GATHER, DUAL>(a, st);
+    if (t.tn == 32) return launch_frag_cfg<T, 2, 2, 4, 1, 2, GATHER, DUAL>(a, st);
+    if (t.tm == 32) return launch_frag_cfg<T, 2, 1, 8, 1, 2, GATHER, DUAL>(a, st);
+    launch_frag_cfg<T, 1, 1, 16, 1, 1, GATHER, DUAL>(a, st);
+}
+
+// bf16: the direct-fragment kernels or the DMA-staged tiles.  Measured times in
+// ns: direct-fragment 4000 + the operand bytes its tiles load from the L2 at
+// 9 KB/ns; staged tiles per round of the CUs 6000 + 640 per 64 of K (1.75 times
+// that for the gather): 512 x 3072 x 768 12.8 against 13.4 us, 999 x 768 x 3072
+// 20.9 against 36, 2048 x 3072 x 768 35 against 16.7.
+static bool frag_faster(const GemmArgs& a, bool gather, BigTile tile, int64_t nsplit) {
+    if (tile == kBigNone) return true;
+    const FragTile t = frag_tile(a.M, a.N, gather, a.Hq);
+    const int64_t bytes = ceil_div(a.M, t.tm) * ceil_div(a.N, t.tn) * (t.tm + t.tn) * a.K * 2;
+    const int64_t bm = tile == kBigSmall || tile == kBigTallS || tile == kBigWide ? 128 : 256;
+    const int64_t per_cu = tile == kBigSmall || tile == kBigTallS ? 2 : 1;
+    const int64_t blocks = ceil_div(a.M, bm) * ceil_div(a.N, big_tile_n(tile)) * nsplit;
+    const int64_t rounds = ceil_div(blocks, per_cu * (int64_t)device_cus());
+    return 4000 + bytes / 9000 < rounds * (6000 + a.K / nsplit * (gather ? 1120 : 640) / 64);
+}
+
+// whether run_gemm gives a bf16 product of more than 64 rows to the
+// direct-fragment kernels
+static bool linear_takes_frag(const GemmArgs& a) {
+    return a.M > 64 && frag_fits<bf16_t, false>(a) &&
+           frag_faster(a, false, big_tile(a.M, a.N, a.K, false, 0), 1);
+}
+
 template <typename T, bool GATHER>
 static int run_gemm(const GemmArgs& a, hipStream_t st, const char* what) {
     if (a.M == 0 || a.N == 0) return LOOM_OK;
@@ -1615,6 +1711,14 @@ static int run_gemm(const GemmArgs& a, hipStream_t st, const char* what) {
                   (uintptr_t)a.src[3] | (uintptr_t)a.src[4]) % 16 == 0;
         else
             sk = sk && a.ldx % 8 == 0 && ((uintptr_t)a.X & 15) == 0;
+        // more than 16 rows: the direct-fragment tiles, which split the rows too
+        // (3072 x 768: M = 32 4.8 -> 4.5 us, 64 6.7 -> 4.9; 768 x 3072: 10.7 ->
+        // 6.6, 16.6 -> 7.0; one 16-row tile: 7.9 us here)
+        if (a.M > 16 && frag_fits<T, GATHER>(a) &&
+            (a.M <= 64 || frag_faster(a, GATHER, big_tile(a.M, a.N, a.K, GATHER, a.Hq), 1))) {
+            launch_frag<T, GATHER, false>(a, st);
+            return launch_status(what);
+        }
         if (sk) {
             const dim3 grid((unsigned)ceil_div(a.N, 16));
             switch ((int)ceil_div(a.M, 16)) {
@@ -1655,6 +1759,12 @@ static int run_gemm(const GemmArgs& a, hipStream_t st, const char* what) {
             gv = gv && a.ldx % 4 == 0 && ((uintptr_t)a.X & 15) == 0;
         if (gv) {
             launch_gemv_f32<GATHER>(a, st);
+            return launch_status(what);
+        }
+        // fp32 on the matrix cores (128 rows: W_real 87 -> 12.7 us, W2 337 ->
+        // 17.3, W_imag 144 -> 18.7)
+        if (frag_fits<T, GATHER>(a)) {
+            launch_frag<T, GATHER, false>(a, st);
             return launch_status(what);
         }
     }
@@ -1804,9 +1914,14 @@ static int linear_multi_dispatch(const loom_linear_multi_desc& d, hipStream_t st
                   ((uintptr_t)d.x & 15) == 0 && g0.ldw % 8 == 0 && g1.ldw % 8 == 0 &&
                   (((uintptr_t)g0.w | (uintptr_t)g1.w) & 15) == 0;
         const BigTile tile = ok ? big_tile(d.m, g0.n + g1.n, d.k, false, 0) : kBigNone;
-        if (tile != kBigNone && g0.n % big_tile_n(tile) == 0) {
-            GemmArgs a{};
-            a.X = d.x; a.ldx = d.ldx; a.W = g0.w; a.ldw = g0.ldw; a.out = g0.out; a.ldc = g0.ldc;
+        GemmArgs a{};
+        a.X = d.x; a.ldx = d.ldx; a.W = g0.w; a.ldw = g0.ldw; a.M = d.m; a.N = g0.n; a.K = d.k;
+        GemmArgs b = a;
+        b.W = g1.w; b.ldw = g1.ldw; b.N = g1.n;
+        // (where a product alone takes the direct-fragment tiles, both run alone:
+        // one launch gives the bits of the separate products)
+        if (tile != kBigNone && g0.n % big_tile_n(tile) == 0 && !linear_takes_frag(a) && !linear_takes_frag(b)) {
+            a.out = g0.out; a.ldc = g0.ldc;
             a.bias = g0.bias; a.gate_p = g0.gate_p; a.gate_alpha = g0.gate_alpha;
             a.M = d.m; a.N = g0.n + g1.n; a.K = d.k;
             a.N1 = g0.n; a.Wb = g1.w; a.ldwb = g1.ldw; a.outb = g1.out; a.ldcb = g1.ldc; a.biasb = g1.bias;
@@ -2036,13 +2151,22 @@ extern "C" int loom_linear_ln(int dtype, const loom_linear_multi_desc* d, const 
                 const int64_t cost = ceil_div(tiles * q, per_cu * (int64_t)device_cus()) * (K / q + 320);
                 if (ns == 0 || cost < best) { ns = q; best = cost; }
             }
+        GemmArgs a{};
+        a.X = d->x; a.ldx = d->ldx; a.W = g.w; a.ldw = g.ldw;
+        a.X2 = d->k2 > 0 ? d->x2 : nullptr; a.ldx2 = d->ldx2; a.W2 = g.w2; a.ldw2 = g.ldw2;
+        a.K1 = d->k;
+        a.M = d->m; a.N = g.n; a.K = K;
+        a.partial = workspace; a.ldp = g.n;
+        // direct-fragment tiles: k split inside a block, one partial sum
+        if (aligned && frag_fits<bf16_t, false>(a) && frag_faster(a, false, ns > 0 ? tile : kBigNone, ns > 0 ? ns : 1)) {
+            if (a.X2 != nullptr) launch_frag<bf16_t, false, true>(a, st);
+            else launch_frag<bf16_t, false, false>(a, st);
+            const int rc = launch_status("loom_linear_ln");
+            if (rc != LOOM_OK) return rc;
+            return launch_splitk_ln(1, d, workspace, gamma, beta, eps, out, ldo, nullptr, st);
+        }
         if (ns > 0) {
-            GemmArgs a{};
-            a.X = d->x; a.ldx = d->ldx; a.W = g.w; a.ldw = g.ldw;
-            a.X2 = d->k2 > 0 ? d->x2 : nullptr; a.ldx2 = d->ldx2; a.W2 = g.w2; a.ldw2 = g.ldw2;
-            a.K1 = d->k;
-            a.M = d->m; a.N = g.n; a.K = K;
-            a.partial = workspace; a.ldp = g.n; a.nsplit = (int)ns;
+            a.nsplit = (int)ns;
             launch_big<false>(a, tile, ns, st);
             const int rc = launch_status("loom_linear_ln");
             if (rc != LOOM_OK) return rc;
@@ -2295,7 +2419,10 @@ extern "C" int loom_prefill_qkv(int dtype, const void* x, int64_t ldx, const voi
                           (uintptr_t)sin_table;
     const uintptr_t a8 = (uintptr_t)q_out | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)hist_out;
     const bool shared = g_shared_tiles.load(std::memory_order_relaxed) != 0;
-    const bool fused = dtype == LOOM_BF16 && HD == 96 && QKV % BgTall::BG_N == 0 &&
+    GemmArgs qkv{};
+    qkv.X = x; qkv.ldx = ldx; qkv.W = w_qkv; qkv.ldw = K; qkv.M = M; qkv.N = QKV; qkv.K = K;
+    // (few rows: the direct-fragment product and the separate RoPE launch)
+    const bool fused = !linear_takes_frag(qkv) && dtype == LOOM_BF16 && HD == 96 && QKV % BgTall::BG_N == 0 &&
                        (shared ? big_fits<BgTallS>(M, K, false, 0) : big_fits<BgTall>(M, K, false, 0)) &&
                        K % 8 == 0 && ldx % 8 == 0 &&
                        (a16 & 15) == 0 && (a8 & 7) == 0 && cache_stride_b % 4 == 0 &&

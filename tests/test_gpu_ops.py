@@ -240,6 +240,44 @@ def test_beta_forward(dtype, QH, HD, Hq, M, sectors):
     assert pack.numel() == 0 and wc.shape == w.shape
 
 
+# each tile of the direct-fragment products (16 x 16, 32 x 16, 32 x 32, 64 x 32,
+# 64 x 64 with eight and with four k parts, and fp32's 128 x 128 blocks), whole
+# and with ragged rows and columns, one unit of k and a k part without work
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("M,N,K", [(17, 64, 64), (33, 40, 192), (47, 1000, 768), (64, 3072, 768), (65, 768, 1536),
+                                   (129, 1500, 768), (255, 768, 3072), (500, 770, 768), (513, 3072, 320),
+                                   (999, 768, 3072), (1000, 3100, 768), (2100, 4000, 64)])
+def test_direct_fragment_products(dtype, M, N, K):
+    from loom_amd import ops
+    g = gen(M + N + K)
+    x, w = dev(rnd(g, M, K), dtype), dev(rnd(g, N, K, scale=K ** -0.5), dtype)
+    bias, p, res = dev(rnd(g, N), torch.float32), dev(rnd(g, M, N), dtype), dev(rnd(g, M, N), dtype)
+    want = (x.double() @ w.double().t()) * (1.0 + 0.2 * p.double()) + bias.double() + res.double()
+    got = ops.linear(x, w, bias, gate_p=p, gate_alpha=0.2, residual=res).double()
+    # fp32 sums of K products: |error| <= K 2^-24 sum |x w| (<= ~K^0.5 here), far from reached;
+    # a bf16 result is rounded once more, by at most 2^-8 of itself
+    bound = 2.0 ** -24 * K * (x.double().abs() @ w.double().abs().t()) * 1.5 + 2.0 ** -20
+    if dtype == torch.bfloat16:
+        bound = bound + 2.0 ** -8 * want.abs()
+    assert bool(((got - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("QH,HD,Hq,M,sectors", [(8, 96, 384, 17, "head"), (8, 96, 384, 65, "open"),
+                                                 (8, 64, 256, 100, "head"), (8, 128, 512, 129, "head"),
+                                                 (2, 32, 48, 33, "head"), (8, 96, 384, 999, "head")])
+def test_direct_fragment_gather(dtype, QH, HD, Hq, M, sectors):
+    from loom_amd import ops
+    N, H = QH * HD, QH * Hq
+    K = ref.imag_in(N, HD, sectors)
+    g = gen(QH + HD + M + Hq)
+    u = dev(rnd(g, 1, M, N), dtype)
+    q, kc, c, d = (dev(rnd(g, 1, M, QH, HD), dtype) for _ in range(4))
+    w = dev(rnd(g, H, K, scale=K ** -0.5), dtype)
+    out = ops.beta_forward_cuda(u, q, kc, c, d, w, Hq, HD, QH, sectors == "open")[0]
+    check(out, ref.beta_space_dense(host(u), host(q), host(kc), host(c), host(d), host(w), QH, HD, sectors), dtype)
+
+
 # ----------------------------------------------------------------- depth attention
 
 @pytest.mark.parametrize("dtype", DTYPES3)
