@@ -664,9 +664,11 @@ gemm_bf16_big_kernel(GemmArgs a) {
 
     // epilogue: output group gi = (i, j) holds the 4 consecutive columns
     // gcol(gi) = ncol + 16i .. +3 of row grow(gi) = mrow + 16j; its bias
-    // operand depends on i only.  Whole tiles take straight-line code with
-    // 8-byte stores (one variant per gate / residual combination, chosen once
-    // per block); edge tiles check every element.
+    // operand depends on i only.  Tiles whole in their columns take straight-line code
+    // (one variant per gate / residual combination, chosen once per block) that
+    // stores the rows below M; tiles with ragged columns check every
+    // element (with ragged rows too checked that way, one such tile made 999 x
+    // 3072 x 768 take 35.7 us, against 13.4 for 512 rows).
     constexpr int NG = FI * FJ;
     constexpr int NB = FI;
     const int64_t mrow = m0 + wm * C::WTM + (lane & 15);
@@ -703,6 +705,9 @@ gemm_bf16_big_kernel(GemmArgs a) {
         });
         return reg;
     };
+    // rows of the wave's tile below M: a staged row past them stores the last
+    // one again (its own bytes, no branch between the LDS reads and the stores)
+    const int rows = (int)min((int64_t)C::WTM, a.M - m0 - wm * C::WTM);
     // regions of BYTES for every wave
     constexpr int REG2 = C::WTM * C::WTN * 2, REG4 = 2 * REG2;
     constexpr bool FIT2 = NS * (KH * XH * 2 / REG2 + KH * WH * 2 / REG2) >= C::WAVES;
@@ -725,9 +730,9 @@ gemm_bf16_big_kernel(GemmArgs a) {
                 if (rot) return (uint16_t*)ro.kc + b * ro.csb + pos * ro.cst + (hd - ro.QH) * ro.csh;
                 return (uint16_t*)ro.vc + b * ro.csb + pos * ro.cst + (hd - ro.QH - ro.KVH) * ro.csh;
             };
-            // staged (16-byte row pieces) when the block's rows are all in range
-            // and every destination row is 16-byte aligned
-            const bool st16 = m0 + BG_M <= a.M && ((ro.csb | ro.cst | ro.csh) & 7) == 0 &&
+            // staged (16-byte row pieces) when every destination row is 16-byte
+            // aligned
+            const bool st16 = ((ro.csb | ro.cst | ro.csh) & 7) == 0 &&
                               (((uintptr_t)ro.q | (uintptr_t)ro.kc | (uintptr_t)ro.vc) & 15) == 0;
             uint16_t* reg = nullptr;
             if (st16) {
@@ -770,11 +775,12 @@ gemm_bf16_big_kernel(GemmArgs a) {
                 }
             }
             if (st16) {
+                if (rows <= 0) return;
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 __builtin_amdgcn_wave_barrier();
 #pragma unroll
                 for (int it = 0; it < C::WTM * 12 / 64; ++it) {
-                    const int c = it * 64 + lane, row = c / 12, pc = c % 12;
+                    const int c = it * 64 + lane, row = min(c / 12, rows - 1), pc = c % 12;
                     *reinterpret_cast<uint4*>(row_dst(m0 + wm * C::WTM + row) + 8 * pc) =
                         *reinterpret_cast<const uint4*>(reg + row * 96 + 8 * (pc ^ ((row >> 1) & 3)));
                 }
@@ -787,8 +793,8 @@ gemm_bf16_big_kernel(GemmArgs a) {
         // columns are in range
         float* part = a.partial + split * a.M * a.ldp;
         if constexpr (FIT4) {
-            if (m0 + BG_M <= a.M && n0 + BG_N <= a.N && (a.ldp & 3) == 0 && ((uintptr_t)part & 15) == 0) {
-                // whole tile, staged: piece p (4 floats) of row r at p ^ (r & 15)
+            if (n0 + BG_N <= a.N && (a.ldp & 3) == 0 && ((uintptr_t)part & 15) == 0) {
+                // whole columns, staged: piece p (4 floats) of row r at p ^ (r & 15)
                 __syncthreads();
                 float* reg = reinterpret_cast<float*>(stage_region(std::integral_constant<int, REG4>{}));
                 constexpr int PR = C::WTN / 4;          // 16-byte pieces of a wave-tile row
@@ -799,12 +805,13 @@ gemm_bf16_big_kernel(GemmArgs a) {
                     *reinterpret_cast<float4*>(reg + rl * C::WTN + 4 * (pc ^ (rl & 15))) =
                         make_float4(gval(gi, 0), gval(gi, 1), gval(gi, 2), gval(gi, 3));
                 }
+                if (rows <= 0) return;
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 __builtin_amdgcn_wave_barrier();
                 float* orow = part + (m0 + wm * C::WTM) * a.ldp + n0 + wn * C::WTN;
 #pragma unroll
                 for (int it = 0; it < C::WTM * PR / 64; ++it) {
-                    const int c = it * 64 + lane, row = c / PR, pc = c % PR;
+                    const int c = it * 64 + lane, row = min(c / PR, rows - 1), pc = c % PR;
                     *reinterpret_cast<float4*>(orow + row * a.ldp + 4 * pc) =
                         *reinterpret_cast<const float4*>(reg + row * C::WTN + 4 * (pc ^ (row & 15)));
                 }
@@ -830,7 +837,9 @@ gemm_bf16_big_kernel(GemmArgs a) {
     const uint16_t* gp = (const uint16_t*)a.gate_p;
     const uint16_t* rs = (const uint16_t*)a.residual;
     const int64_t ldc = a.ldc;
-    const bool whole = m0 + BG_M <= a.M && n0 + BG_N <= a.N && (ldc & 3) == 0 &&
+    // tiles whole in their columns (rows past M are not stored; their operand
+    // loads read the last row)
+    const bool whole = n0 + BG_N <= a.N && (ldc & 3) == 0 &&
                        (((uintptr_t)out | (uintptr_t)gp | (uintptr_t)rs) & 7) == 0 &&
                        ((uintptr_t)a.bias & 15) == 0;
     auto bf4 = [](uint2 w, float (&x)[4]) {
@@ -857,7 +866,7 @@ gemm_bf16_big_kernel(GemmArgs a) {
                                        : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int gi = 0; gi < NG; ++gi) {
-            const int64_t e = grow(gi) * ldc + gcol(gi);
+            const int64_t e = min(grow(gi), a.M - 1) * ldc + gcol(gi);
             if constexpr (GATE) gw[gi] = *reinterpret_cast<const uint2*>(gp + e);
             if constexpr (RES) rw[gi] = *reinterpret_cast<const uint2*>(rs + e);
         }
@@ -881,18 +890,19 @@ gemm_bf16_big_kernel(GemmArgs a) {
                 const int rl = 16 * (gi % FJ) + (lane & 15);             // row of the wave tile
                 const int cl = 16 * gslot(gi) + (lane >> 4) * 4;         // column of the wave tile
                 *reinterpret_cast<uint2*>(reg + rl * C::WTN + 8 * ((cl >> 3) ^ ((rl >> 1) & 3)) + (cl & 7)) = w;
-            } else {
+            } else if (grow(gi) < a.M) {
                 *reinterpret_cast<uint2*>(out + e) = w;
             }
         }
         if (staged) {
+            if (rows <= 0) return;
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
             constexpr int PR = C::WTN / 8;  // 16-byte pieces of a wave-tile row
             uint16_t* orow = out + (m0 + wm * C::WTM) * ldc + n0 + wn * C::WTN;
 #pragma unroll
             for (int it = 0; it < C::WTM * PR / 64; ++it) {
-                const int c = it * 64 + lane, row = c / PR, pc = c % PR;
+                const int c = it * 64 + lane, row = min(c / PR, rows - 1), pc = c % PR;
                 const uint4 v = *reinterpret_cast<const uint4*>(reg + row * C::WTN + 8 * (pc ^ ((row >> 1) & 3)));
                 *reinterpret_cast<uint4*>(orow + row * ldc + 8 * pc) = v;
             }
@@ -1612,21 +1622,28 @@ static void launch_big(const GemmArgs& a, BigTile tile, int64_t nsplit, hipStrea
     }
 }
 
-// Wave tile of a direct-fragment product (gemm_frag.h): the largest that still
-// gives 3/4 of the CUs a block and does not pad M to twice its rows.  Measured
-// over M = 32 .. 2048 at 768 x 768, 3072 x 768, 768 x 3072 and the W_imag
-// gather, that tile was the fastest or within 5% of it in both types (bf16
-// 768 x 3072: M = 64 7.0 us in 16 x 16 tiles, 128 9.2 in 32 x 16, 256 11.1 in
-// 32 x 32, 512 15.0 in 64 x 32, 999 20.9 in 64 x 64; the neighbouring sizes
-// 8.5, 10.8, 15.0, 18.7, 27.7).
-struct FragTile { int tm, tn; };
-static FragTile frag_tile(int64_t M, int64_t N, bool gather, int64_t Hq) {
-    static constexpr FragTile kTiles[] = {{64, 64}, {64, 32}, {32, 32}, {32, 16}};
-    for (const FragTile& t : kTiles)
-        if (2 * M > t.tm && (!gather || Hq % t.tn == 0) &&
-            4 * ceil_div(M, t.tm) * ceil_div(N, t.tn) >= 3 * (int64_t)device_cus())
-            return t;
-    return FragTile{16, 16};
+// Wave tile of a direct-fragment product (gemm_frag.h) and its estimated time in
+// ns: 3000 + per round of the CUs the operand bytes of a tile at 48 bytes/ns (a
+// CU's rate from the L2), and in fp32 half the time of its MFMAs at 614
+// flop/ns.  bf16, measured (estimated) us: 768 x 3072 with M = 64 in 16 x 16
+// tiles 7.0 (7.1), 128 in 32 x 16 9.2 (9.1), 256 in 32 x 32 11.1 (11.2), 512
+// in 64 x 32 15.0 (15.3), 999 in 64 x 64 20.9 (19.4), the neighbouring sizes
+// 8.5, 10.8, 15.0, 18.7, 27.7; fp32 M = 64 11.9 (12.4), 256 25.3 (24.4), 999
+// 54 (56).
+struct FragTile { int tm, tn; int64_t ns; };
+template <typename T>
+static FragTile frag_tile(int64_t M, int64_t N, int64_t K, bool gather, int64_t Hq) {
+    static constexpr int kTiles[][2] = {{16, 16}, {32, 16}, {32, 32}, {64, 32}, {64, 64}};
+    FragTile best{16, 16, INT64_MAX};
+    for (const auto& t : kTiles) {
+        const int64_t tm = t[0], tn = t[1];
+        if (gather && Hq % tn != 0) continue;
+        const int64_t rounds = ceil_div(ceil_div(M, tm) * ceil_div(N, tn), (int64_t)device_cus());
+        const int64_t mfma = sizeof(T) == 4 ? tm * tn * K / 614 : 0;
+        const int64_t ns = 3000 + rounds * ((tm + tn) * K * (int64_t)sizeof(T) / 48 + mfma);
+        if (ns < best.ns) best = FragTile{(int)tm, (int)tn, ns};
+    }
+    return best;
 }
 
 // What the direct-fragment kernels need of a product: whole units of k, 16-byte
@@ -1650,47 +1667,39 @@ static bool frag_fits(const GemmArgs& a) {
     return ok;
 }
 
-template <typename T, int MT, int NT, int KW, int SP, int U, bool GATHER, bool DUAL>
+template <typename T, int MT, int NT, int KW, int U, bool GATHER, bool DUAL>
 static void launch_frag_cfg(const GemmArgs& a, hipStream_t st) {
-    using C = FragCfg<T, MT, NT, KW, SP, U>;
-    const dim3 grid((unsigned)(ceil_div(a.M, C::BM) * ceil_div(a.N, C::BN)));
-    hipLaunchKernelGGL((gemm_frag_kernel<T, MT, NT, KW, SP, U, GATHER, DUAL>), grid, dim3(C::THREADS), 0, st, a);
+    using C = FragCfg<T, MT, NT, KW, U>;
+    const dim3 grid((unsigned)(ceil_div(a.M, C::TM) * ceil_div(a.N, C::TN)));
+    hipLaunchKernelGGL((gemm_frag_kernel<T, MT, NT, KW, U, GATHER, DUAL>), grid, dim3(C::THREADS), 0, st, a);
 }
 template <typename T, bool GATHER, bool DUAL>
 static void launch_frag(const GemmArgs& a, hipStream_t st) {
-    const FragTile t = frag_tile(a.M, a.N, GATHER, a.Hq);
-    constexpr bool F32 = sizeof(T) == 4;
+    const FragTile t = frag_tile<T>(a.M, a.N, a.K, GATHER, a.Hq);
     if (t.tm == 64 && t.tn == 64) {
         // eight k parts (one block per CU) or four (two blocks per CU), whichever
-        // fills its rounds better; many fp32 tiles: 2 x 2 waves per block and no
-        // k split (4096 x 3072 x 768: 182 against 215 us)
+        // fills its rounds better
         const int64_t n = ceil_div(a.M, 64) * ceil_div(a.N, 64), c = device_cus();
-        if constexpr (F32 && !DUAL) {
-            if (n >= 8 * c && (!GATHER || a.Hq % 128 == 0)) return launch_frag_cfg<T, 4, 4, 1, 2, 1, GATHER, DUAL>(a, st);
-        }
-        if (n <= c || ceil_div(n, c) < 2 * ceil_div(n, 2 * c)) return launch_frag_cfg<T, 4, 4, 8, 1, 1, GATHER, DUAL>(a, st);
-        return launch_frag_cfg<T, 4, 4, 4, 1, 1, GATHER, DUAL>(a, st);
+        if (n <= c || ceil_div(n, c) < 2 * ceil_div(n, 2 * c)) return launch_frag_cfg<T, 4, 4, 8, 1, GATHER, DUAL>(a, st);
+        return launch_frag_cfg<T, 4, 4, 4, 1, GATHER, DUAL>(a, st);
     }
-    if (t.tm == 64) return launch_frag_cfg<T, 4, 2, F32 ? 4 : 8, 1, 1, GATHER, DUAL>(a, st);
-    if (t.tn == 32) return launch_frag_cfg<T, 2, 2, 4, 1, 2, GATHER, DUAL>(a, st);
-    if (t.tm == 32) return launch_frag_cfg<T, 2, 1, 8, 1, 2, GATHER, DUAL>(a, st);
-    launch_frag_cfg<T, 1, 1, 16, 1, 1, GATHER, DUAL>(a, st);
+    if (t.tm == 64) return launch_frag_cfg<T, 4, 2, sizeof(T) == 4 ? 4 : 8, 1, GATHER, DUAL>(a, st);
+    if (t.tn == 32) return launch_frag_cfg<T, 2, 2, 4, 2, GATHER, DUAL>(a, st);
+    if (t.tm == 32) return launch_frag_cfg<T, 2, 1, 8, 2, GATHER, DUAL>(a, st);
+    launch_frag_cfg<T, 1, 1, 16, 1, GATHER, DUAL>(a, st);
 }
 
-// bf16: the direct-fragment kernels or the DMA-staged tiles.  Measured times in
-// ns: direct-fragment 4000 + the operand bytes its tiles load from the L2 at
-// 9 KB/ns; staged tiles per round of the CUs 6000 + 640 per 64 of K (1.75 times
-// that for the gather): 512 x 3072 x 768 12.8 against 13.4 us, 999 x 768 x 3072
-// 20.9 against 36, 2048 x 3072 x 768 35 against 16.7.
+// bf16: the direct-fragment kernels or the DMA-staged tiles, by the estimate
+// above and, for the staged tiles, per round of the CUs 6000 ns + 640 per 64 of
+// K (1120 for the gather).  Measured: 999 x 768 x 3072 20.9 against 37 us, 512 x
+// 3072 x 768 12.0 against 13.4, 2048 x 3072 x 768 35 against 16.6.
 static bool frag_faster(const GemmArgs& a, bool gather, BigTile tile, int64_t nsplit) {
     if (tile == kBigNone) return true;
-    const FragTile t = frag_tile(a.M, a.N, gather, a.Hq);
-    const int64_t bytes = ceil_div(a.M, t.tm) * ceil_div(a.N, t.tn) * (t.tm + t.tn) * a.K * 2;
     const int64_t bm = tile == kBigSmall || tile == kBigTallS || tile == kBigWide ? 128 : 256;
     const int64_t per_cu = tile == kBigSmall || tile == kBigTallS ? 2 : 1;
     const int64_t blocks = ceil_div(a.M, bm) * ceil_div(a.N, big_tile_n(tile)) * nsplit;
     const int64_t rounds = ceil_div(blocks, per_cu * (int64_t)device_cus());
-    return 4000 + bytes / 9000 < rounds * (6000 + a.K / nsplit * (gather ? 1120 : 640) / 64);
+    return frag_tile<bf16_t>(a.M, a.N, a.K, gather, a.Hq).ns < rounds * (6000 + a.K / nsplit * (gather ? 1120 : 640) / 64);
 }
 
 // whether run_gemm gives a bf16 product of more than 64 rows to the

@@ -23,35 +23,29 @@ namespace loom {
 // the matrix cores, where the exchange costs more than it saves (256 x 768 x
 // 3072 31 -> 44 us), and take the plain order.
 //
-// U: units of operands in flight per wave.  SP: the block is SP x SP waves of
-// one k part each instead (no LDS, no barrier).
-template <typename T, int MT, int NT, int KW, int SP, int U>
+// U: units of operands in flight per wave.
+template <typename T, int MT, int NT, int KW, int U>
 struct FragCfg {
     static constexpr int TM = 16 * MT, TN = 16 * NT;      // wave tile
-    static constexpr int BM = TM * SP, BN = TN * SP;      // block tile
-    static constexpr int THREADS = 64 * KW * SP * SP;
+    static constexpr int THREADS = 64 * KW;
     static constexpr int CK = 64 / (int)sizeof(T);        // k per chunk
     static constexpr bool SWAP = sizeof(T) == 2 || MT * NT <= 2;
-    static_assert(KW == 1 || SP == 1, "either the waves split K or the tile");
 };
 // k per unit: K (and K1 of a second input) must be a multiple
 template <typename T> constexpr int kFragK = 128 / (int)sizeof(T);
 
-template <typename T, int MT, int NT, int KW, int SP, int U, bool GATHER, bool DUAL>
-__global__ void __launch_bounds__(64 * KW * SP * SP)
+template <typename T, int MT, int NT, int KW, int U, bool GATHER, bool DUAL>
+__global__ void __launch_bounds__(64 * KW)
 gemm_frag_kernel(GemmArgs a) {
-    using C = FragCfg<T, MT, NT, KW, SP, U>;
+    using C = FragCfg<T, MT, NT, KW, U>;
     constexpr int E = (int)sizeof(T);
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int kw = KW > 1 ? wave : 0;
+    const int kw = __builtin_amdgcn_readfirstlane(tid >> 6);
     // the m-tiles of one n-tile are neighbours on one XCD (they share the W
     // rows in its L2; X is the smaller operand in the products this serves)
-    const int MTL = (int)ceil_div(a.M, C::BM);
+    const int MTL = (int)ceil_div(a.M, C::TM);
     const int b = xcd_contiguous((int)blockIdx.x, (int)gridDim.x);
-    const int64_t n0 = (int64_t)(b / MTL) * C::BN + (SP > 1 ? (wave / SP) * C::TN : 0);
-    const int64_t m0 = (int64_t)(b % MTL) * C::BM + (SP > 1 ? (wave % SP) * C::TM : 0);
-    if (SP > 1 && (m0 >= a.M || n0 >= a.N)) return;       // no barrier in the SP form
+    const int64_t n0 = (int64_t)(b / MTL) * C::TN, m0 = (int64_t)(b % MTL) * C::TM;
     const int64_t g = GATHER ? n0 / a.Hq : 0;
     const int64_t ldx = GATHER ? a.Nm : a.ldx;
     const int fr = lane & 15, fq = lane >> 4;
@@ -211,37 +205,29 @@ gemm_frag_kernel(GemmArgs a) {
                 if (nb + r < a.N) st(op + r, epilogue<T>(a, m, nb + r, v[r]));
         }
     };
-    if constexpr (KW == 1) {
+    // partial tiles to LDS: the float4 of lane (fr, fq) of tile (i, j) at
+    // slot fr ^ (4*fq + i) of its 16, so that the sum below, which reads
+    // row runs (consecutive threads: consecutive columns), spreads over
+    // the banks
+    __shared__ __attribute__((aligned(16))) f32x4 red[KW][NT * MT * 64];
 #pragma unroll
-        for (int i = 0; i < NT; ++i)
+    for (int i = 0; i < NT; ++i)
 #pragma unroll
-            for (int j = 0; j < MT; ++j)
-                store4(m0 + 16 * j + fr, n0 + 16 * i + 4 * fq, acc[i][j]);
-    } else {
-        // partial tiles to LDS: the float4 of lane (fr, fq) of tile (i, j) at
-        // slot fr ^ (4*fq + i) of its 16, so that the sum below, which reads
-        // row runs (consecutive threads: consecutive columns), spreads over
-        // the banks
-        __shared__ __attribute__((aligned(16))) f32x4 red[KW][NT * MT * 64];
+        for (int j = 0; j < MT; ++j)
+            red[kw][(i * MT + j) * 64 + fq * 16 + (fr ^ ((4 * fq + i) & 15))] = acc[i][j];
+    __syncthreads();
+    constexpr int NQ = C::TN / 4;                     // float4 columns of a row
+    constexpr int TOT = C::TM * NQ;
 #pragma unroll
-        for (int i = 0; i < NT; ++i)
+    for (int it = 0; it < (TOT + C::THREADS - 1) / C::THREADS; ++it) {
+        const int q = it * C::THREADS + tid;
+        if (TOT % C::THREADS != 0 && q >= TOT) break;
+        const int m = q / NQ, n4 = q % NQ, i = n4 >> 2, gq = n4 & 3;
+        const int at = (i * MT + (m >> 4)) * 64 + gq * 16 + ((m & 15) ^ ((4 * gq + i) & 15));
+        f32x4 s = red[0][at];
 #pragma unroll
-            for (int j = 0; j < MT; ++j)
-                red[kw][(i * MT + j) * 64 + fq * 16 + (fr ^ ((4 * fq + i) & 15))] = acc[i][j];
-        __syncthreads();
-        constexpr int NQ = C::TN / 4;                     // float4 columns of a row
-        constexpr int TOT = C::TM * NQ;
-#pragma unroll
-        for (int it = 0; it < (TOT + C::THREADS - 1) / C::THREADS; ++it) {
-            const int q = it * C::THREADS + tid;
-            if (TOT % C::THREADS != 0 && q >= TOT) break;
-            const int m = q / NQ, n4 = q % NQ, i = n4 >> 2, gq = n4 & 3;
-            const int at = (i * MT + (m >> 4)) * 64 + gq * 16 + ((m & 15) ^ ((4 * gq + i) & 15));
-            f32x4 s = red[0][at];
-#pragma unroll
-            for (int w = 1; w < KW; ++w) s += red[w][at];
-            store4(m0 + m, n0 + 4 * n4, s);
-        }
+        for (int w = 1; w < KW; ++w) s += red[w][at];
+        store4(m0 + m, n0 + 4 * n4, s);
     }
 }
 

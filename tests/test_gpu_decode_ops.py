@@ -247,6 +247,39 @@ def _prefill_qkv_case(dtype, B, Tc, start, HD, hist):
     assert not kc[:, :, :start].any() and not kc[:, :, start + Tc:].any()
 
 
+@pytest.mark.parametrize("shared", [False, True])
+@pytest.mark.parametrize("M", [2047, 3131, 4001])
+def test_staged_tiles_with_ragged_rows(M, shared):
+    """The DMA-staged tiles store a last row tile with rows missing as they
+    store a whole one (row-masked): plain, gated + residual, split-K +
+    LayerNorm and RoPE epilogues; nothing is written past row M."""
+    from loom_amd import _lib, ops
+    bf, K, N = torch.bfloat16, 768, 768
+    g = torch.Generator().manual_seed(M)
+    r = lambda *s, sc=1.0: (torch.randn(*s, generator=g) * sc).to(DEV, bf)
+    x, w, p, res = r(M, K), r(N, K, sc=K ** -0.5), r(M, N), r(M, N)
+    bias, gam, bet = (torch.randn(N, generator=g).to(DEV) for _ in range(3))
+    want = host(x) @ host(w).T
+    nb = _lib.load().loom_linear_ln_workspace_bytes(M, N)
+    ws = torch.empty(nb // 4, device=DEV)
+    with shared_tiles(shared):
+        for kw, ref_ in ((dict(), want), (dict(gate_p=p, gate_alpha=0.2, residual=res),
+                                          want * (1 + 0.2 * host(p)) + host(res))):
+            out = torch.full((M + 3, N), 7.0, device=DEV, dtype=bf)
+            ops.linear(x, w, bias, out=out[:M], **kw)
+            check(out[:M], ref_ + host(bias), bf)
+            assert bool((out[M:] == 7.0).all())
+        y, out = torch.zeros(M, N, device=DEV, dtype=bf), torch.full((M + 3, N), 7.0, device=DEV, dtype=bf)
+        d = _lib.linear_multi_desc(x, [dict(w=w, w2=w, out=y, bias=bias)], x2=p)
+        _lib.call("loom_linear_ln", code(x), ctypes.byref(d), P(gam), P(bet), 1e-5, P(out), N, P(ws), nb, None, S(x))
+        check(out[:M], torch.nn.functional.layer_norm(want + host(p) @ host(w).T + host(bias), (N,), host(gam),
+                                                      host(bet), 1e-5), bf)
+        assert bool((out[M:] == 7.0).all())
+    if M == 3131:
+        with shared_tiles(shared):
+            _prefill_qkv_case(bf, 31, 101, 5, 96, True)
+
+
 @contextlib.contextmanager
 def shared_tiles(on):
     """The library's shared-tile mode set for the block, restored after."""

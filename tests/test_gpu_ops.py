@@ -241,7 +241,7 @@ def test_beta_forward(dtype, QH, HD, Hq, M, sectors):
 
 
 # each tile of the direct-fragment products (16 x 16, 32 x 16, 32 x 32, 64 x 32,
-# 64 x 64 with eight and with four k parts, and fp32's 128 x 128 blocks), whole
+# 64 x 64 with eight and with four k parts), whole
 # and with ragged rows and columns, one unit of k and a k part without work
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("M,N,K", [(17, 64, 64), (33, 40, 192), (47, 1000, 768), (64, 3072, 768), (65, 768, 1536),
