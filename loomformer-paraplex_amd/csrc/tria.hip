@@ -1341,8 +1341,11 @@ final_ca_row_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* _
         lse[row] = red[0] == -INFINITY ? -INFINITY : red[0] + logf(red[1]);
 }
 
-// ---------------------------------------------------------------- dispatch
+}  // namespace loom
+#include "final_ca_tile.h"
+namespace loom {
 
+// ---------------------------------------------------------------- dispatch
 template <typename T>
 static int tria_depth_dispatch(const void* r, const void* i, const void* o, const void* prev,
                                const void* seed, const uint8_t* valid, const void* w,
@@ -1523,6 +1526,18 @@ static int polarm_dispatch(const void* in, void* out, const uint8_t* mask, int64
     return launch_status("loom_polarm_forward");
 }
 
+// The 16-row tiles of a sequence against one block per row, measured at D =
+// 768: bf16 from more rows than CUs on (256 rows of 16 keys 5.6 us against 5.7,
+// 512 9.5 against 6.0, 16384 of 15 255 against 15.3; the one-row kernel holds a
+// row of up to 64 keys in registers, two blocks per CU); fp32, whose one-row
+// blocks run eight per CU, from rows x keys of 32 K on (14 K 8.5 us against 9.5,
+// 127 K 38 against 16, 245 K 80 against 31).
+template <typename T>
+static bool ca_tiles_faster(int64_t rows, int64_t T_, int64_t K) {
+    if (T_ <= 1) return false;
+    return sizeof(T) == 2 ? rows > (int64_t)device_cus() : rows * K >= 32768;
+}
+
 template <typename T>
 static int final_ca_dispatch(const void* q, const void* k, const void* v, int64_t kv_stride_b,
                              const uint8_t* allowed, int64_t allowed_stride, const void* residual,
@@ -1531,6 +1546,24 @@ static int final_ca_dispatch(const void* q, const void* k, const void* v, int64_
     const bool vec = D % 8 == 0 && D <= kCaChunks * 64 * 8 && kv_stride_b % 8 == 0 &&
                      (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out |
                        (uintptr_t)residual) & 15) == 0;
+    if constexpr (!std::is_same<T, f16_t>::value) {
+        // 16 query rows per block
+        if (vec && D % 64 == 0 && D <= 256 * kCaTileMaxSlabs && K >= 1 && K <= 256 && ca_tiles_faster<T>(B * T_, T_, K)) {
+            const dim3 grid((unsigned)(B * ceil_div(T_, kCaTileRows)));
+            const int ns = D <= 512 ? 2 : D <= 768 ? 3 : 4;
+#define LOOM_CA_TILE(NKT, NS)                                                                    \
+            if (K <= 16 * NKT && ns == NS) {                                                     \
+                hipLaunchKernelGGL((final_ca_tile_kernel<T, NKT, NS>), grid, dim3(256), 0, st, (const T*)q, \
+                                   (const T*)k, (const T*)v, kv_stride_b, allowed, allowed_stride, \
+                                   (const T*)residual, gamma, (T*)out, lse, T_, K, k_dev, (int)D, scale); \
+                return launch_status("loom_final_ca_sparse_forward");                            \
+            }
+#define LOOM_CA_TILES(NKT) LOOM_CA_TILE(NKT, 2) LOOM_CA_TILE(NKT, 3) LOOM_CA_TILE(NKT, 4)
+            LOOM_CA_TILES(1) LOOM_CA_TILES(2) LOOM_CA_TILES(4) LOOM_CA_TILES(16)
+#undef LOOM_CA_TILES
+#undef LOOM_CA_TILE
+        }
+    }
     if constexpr (sizeof(T) == 2) {
         if (vec && K <= kCaRowKeys && D <= 1024) {
             hipLaunchKernelGGL((final_ca_row_kernel<T>), dim3((unsigned)(B * T_)), dim3(512), 0, st,

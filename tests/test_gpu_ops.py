@@ -765,6 +765,52 @@ def test_polarm_and_final_ca(dtype):
     check(lse[ok.to(DEV)], wl[ok], torch.float32, rtol=1e-3, atol=1e-3)
 
 
+# the 16-row tiles of the sequence form: 1 to 16 key tiles (and one key more than
+# a tile), ragged rows, 1 to 4 slabs per wave, and the widths and key counts that
+# stay with the one-row kernels (D = 1536, 96 and 1100)
+@pytest.mark.parametrize("dtype", DTYPES3)
+@pytest.mark.parametrize("B,T,K,D", [(150, 2, 1, 64), (130, 17, 15, 768), (70, 33, 16, 512), (16, 130, 17, 1024),
+                                     (26, 40, 33, 320), (12, 31, 100, 768), (9, 16, 256, 128), (1, 300, 120, 256),
+                                     (60, 5, 9, 1536), (20, 20, 9, 96), (20, 20, 9, 1100)])
+def test_final_ca_sequences(dtype, B, T, K, D):
+    from loom_amd import ops
+    g = gen(B + T + K + D)
+    q, k, v = dev(rnd(g, B, T, D), dtype), dev(rnd(g, B, K, D), dtype), dev(rnd(g, B, K, D), dtype)
+    allowed = torch.rand(B, T, K, generator=g) > 0.4
+    allowed[0, T // 2] = False
+    out, lse = ops.final_ca_sparse_forward(q, k, v, dev(allowed, torch.bool), D ** -0.5)
+    check(out, ref.final_ca_sparse(host(q), host(k), host(v), allowed, D ** -0.5), dtype)
+    assert torch.all(host(out)[0, T // 2] == 0) and float(lse[0, T // 2]) == -math.inf
+    wl = ref.final_ca_sparse_lse(host(q), host(k), host(v), allowed, D ** -0.5)
+    ok = allowed.any(-1)
+    check(lse[ok.to(DEV)], wl[ok], torch.float32, rtol=1e-3, atol=1e-3)
+
+
+def test_final_ca_tiles_strided_with_device_key_count():
+    """The 16-row tiles through the cache layout: padded strides, a residual, the
+    key count on the device (also zero keys), values past it never read into a row."""
+    from loom_amd import _lib
+    B, T, cap, D, P = 90, 19, 20, 768, _lib.ptr
+    for dtype in DTYPES:
+        g = gen(5)
+        q, res = dev(rnd(g, B, T, D), dtype), dev(rnd(g, B, T, D), dtype)
+        kb, vb = dev(rnd(g, B, cap + 2, D), dtype), dev(rnd(g, B, cap + 2, D), dtype)
+        al = torch.rand(B, T, cap + 4, generator=g) > 0.3
+        ald = al.to(DEV).to(torch.uint8)
+        for n in (0, 7, 20):
+            kn, vn = kb.clone(), vb.clone()
+            kn[:, n:], vn[:, n:] = float("nan"), float("inf")
+            cnt, out = torch.tensor([n], device=DEV), torch.empty_like(q)
+            _lib.call("loom_final_ca_sparse_strided", _lib.DTYPE_CODE[dtype], P(q), P(kn), P(vn), (cap + 2) * D,
+                      P(ald), cap + 4, P(res), 0.3, P(out), None, B, T, cap, P(cnt), D, D ** -0.5,
+                      _lib.stream_of(q))
+            want = host(res)
+            if n:
+                want = want + 0.3 * ref.final_ca_sparse(host(q), host(kb[:, :n]), host(vb[:, :n]), al[:, :, :n],
+                                                        D ** -0.5)
+            check(out, want, dtype)
+
+
 # ----------------------------------------------------------------- drop-in
 
 def test_drop_in_build_or_load_runs_on_gpu():
