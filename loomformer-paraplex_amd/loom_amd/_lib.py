@@ -131,6 +131,7 @@ QUERIES = {"loom_gqa_workspace_bytes": ([c_int64] * 5, c_int64),
 
 _lib = None
 _lock = threading.Lock()
+_raw_stream = torch._C._cuda_getCurrentRawStream
 
 DTYPE_CODE = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 
@@ -167,7 +168,7 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
 
 def call(name: str, *args) -> None:
     """Call an entry point; raise RuntimeError(loom_last_error()) on failure."""
-    lib = load()
+    lib = _lib or load()
     rc = getattr(lib, name)(*args)
     if rc != 0:
         msg = lib.loom_last_error().decode("utf-8", "replace")
@@ -257,6 +258,17 @@ def frag_major(x: torch.Tensor) -> torch.Tensor:
     xp[:m] = x
     # [j, r, s, q, e] -> [j, s, q, r, e]: piece (j, s, l = r + 16 q) holds row 16j + r, cols 32s + 8q ..
     return xp.view(mp // 16, 16, k // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous().view(-1)
+
+
+def addr(t):
+    """Device address of a tensor as an int (None -> NULL), for the declared
+    pointer arguments of the library's functions."""
+    return None if t is None else t.data_ptr()
+
+
+def raw_stream(device) -> int:
+    """Handle of the current stream of a tensor's device (an int)."""
+    return _raw_stream(device.index)
 
 
 def ptr(t):

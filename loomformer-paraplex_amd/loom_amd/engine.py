@@ -35,7 +35,7 @@ from . import _lib
 from .config import ModelConfig
 from .weights import rope_tables
 
-_P = _lib.ptr
+_P = _lib.addr
 
 
 class LoomDecoder:
@@ -222,7 +222,7 @@ class LoomDecoder:
             raise RuntimeError(self.lib.loom_last_error().decode())
 
     def _stream(self):
-        return _lib.c_void_p(torch.cuda.current_stream(self.dev).cuda_stream)
+        return torch.cuda.current_stream(self.dev).cuda_stream
 
     def wo_for(self, sub: int) -> torch.Tensor:
         """The depth readout of sublayer `sub` (DepthAttn.forward, loomformer.py:3424-3428)."""

@@ -16,7 +16,7 @@ from typing import List, Optional, Sequence, Tuple
 import torch
 
 from . import _lib
-from ._lib import call, dtype_code, ptr, stream_of
+from ._lib import addr, call, dtype_code, raw_stream
 
 _FLOATS = (torch.float32, torch.bfloat16, torch.float16)
 
@@ -27,14 +27,22 @@ def _check(cond: bool, msg: str) -> None:
 
 
 def _cuda(*ts, name: str) -> None:
-    _check(all(t.is_cuda for t in ts), f"{name}: all inputs must be CUDA tensors")
-    dev = ts[0].device
-    _check(all(t.device == dev for t in ts), f"{name}: all inputs must be on the same CUDA device")
+    dev = ts[0].get_device()
+    for t in ts:
+        if not t.is_cuda:
+            raise RuntimeError(f"{name}: all inputs must be CUDA tensors")
+    for t in ts:
+        if t.get_device() != dev:
+            raise RuntimeError(f"{name}: all inputs must be on the same CUDA device")
 
 
 def _same_dtype(*ts, name: str) -> None:
-    _check(all(t.dtype == ts[0].dtype for t in ts), f"{name}: all inputs must have the same dtype")
-    _check(ts[0].dtype in _FLOATS, f"{name}: unsupported dtype {ts[0].dtype}")
+    dt = ts[0].dtype
+    for t in ts:
+        if t.dtype != dt:
+            raise RuntimeError(f"{name}: all inputs must have the same dtype")
+    if dt not in _FLOATS:
+        raise RuntimeError(f"{name}: unsupported dtype {dt}")
 
 
 def _c(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
@@ -46,33 +54,33 @@ def _c(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
 def paraplex_forward(p_real, gate_src, beta_linear, bias, trace, trace_w, reset, anchor,
                      mode: int, update_anchor: bool, decay: float, m: float) -> List[torch.Tensor]:
     """kernels/paraplex/paraplex_launcher.cu:49 (checks :16-47)."""
-    _check(all(t.is_cuda for t in (p_real, gate_src, beta_linear, bias, trace, trace_w, anchor)),
-           "paraplex: CUDA tensors required")
+    _check(p_real.is_cuda and gate_src.is_cuda and beta_linear.is_cuda and bias.is_cuda and trace.is_cuda
+           and trace_w.is_cuda and anchor.is_cuda, "paraplex: CUDA tensors required")
     dev = p_real.device
-    _check(all(t.device == dev for t in (gate_src, beta_linear, bias, trace, trace_w, anchor)),
+    idx = dev.index
+    _check(gate_src.get_device() == idx and beta_linear.get_device() == idx and bias.get_device() == idx
+           and trace.get_device() == idx and trace_w.get_device() == idx and anchor.get_device() == idx,
            "paraplex: device mismatch")
-    _check(p_real.dim() == 3 and beta_linear.shape == p_real.shape and gate_src.shape == p_real.shape,
+    shape, dt = p_real.shape, p_real.dtype
+    _check(len(shape) == 3 and beta_linear.shape == shape and gate_src.shape == shape,
            "p/gate_src/beta must be [B,T,H]")
-    _check(gate_src.dtype == p_real.dtype,
+    _check(gate_src.dtype == dt,
            "paraplex: gate_src dtype must match p_real (cast before calling, same as beta_linear)")
-    _check(beta_linear.dtype == p_real.dtype and trace.dtype == p_real.dtype,
-           "p/beta/trace dtype mismatch")
-    _check(trace.dim() == 2 and trace.shape[0] == p_real.shape[0] and trace.shape[1] == p_real.shape[2],
-           "trace must be [B,H]")
+    _check(beta_linear.dtype == dt and trace.dtype == dt, "p/beta/trace dtype mismatch")
+    B, T, H = shape
+    _check(trace.dim() == 2 and trace.shape[0] == B and trace.shape[1] == H, "trace must be [B,H]")
     _check(bias.dtype == torch.float32 and trace_w.dtype == torch.float32 and anchor.dtype == torch.float32,
            "bias/trace_w/anchor must be float32")
-    _check(bias.numel() == p_real.shape[2] and trace_w.numel() == p_real.shape[2] and anchor.numel() == 1,
-           "parameter shape mismatch")
-    _check(reset.numel() == 0 or (reset.is_cuda and reset.dtype == torch.bool and reset.dim() == 2
-                                  and reset.shape[0] == p_real.shape[0] and reset.shape[1] == p_real.shape[1]),
-           "reset must be empty or bool [B,T]")
-    _check(reset.numel() == 0 or reset.device == dev, "reset device mismatch")
+    _check(bias.numel() == H and trace_w.numel() == H and anchor.numel() == 1, "parameter shape mismatch")
+    has_reset = reset.numel() != 0
+    _check(not has_reset or (reset.is_cuda and reset.dtype == torch.bool and reset.dim() == 2
+                             and reset.shape[0] == B and reset.shape[1] == T), "reset must be empty or bool [B,T]")
+    _check(not has_reset or reset.device == dev, "reset device mismatch")
     _check(p_real.numel() > 0, "paraplex: empty tensors are unsupported")
-    _check(p_real.dtype in _FLOATS, f"paraplex: unsupported dtype {p_real.dtype}")
+    _check(dt in _FLOATS, f"paraplex: unsupported dtype {dt}")
     if update_anchor:
         raise RuntimeError("paraplex: the secant-anchor EMA update is training-only and not "
                            "supported by the inference library (update_anchor must be False)")
-    B, T, H = p_real.shape
     pc = p_real.contiguous()
     gc = pc if gate_src is p_real else gate_src.contiguous()
     bc = beta_linear.contiguous()
@@ -80,12 +88,12 @@ def paraplex_forward(p_real, gate_src, beta_linear, bias, trace, trace_w, reset,
     s = torch.empty_like(pc)
     nxt = torch.empty(B, H, dtype=pc.dtype, device=dev)
     snap = torch.empty(anchor.shape, dtype=torch.float32, device=dev)
-    rc = reset.contiguous() if reset.numel() else None
+    rc = reset.contiguous() if has_reset else None
     # contiguous copies are bound to names so they outlive the asynchronous launch
-    bias_c, trace_c, tw_c, anchor_c = (t.contiguous() for t in (bias, trace, trace_w, anchor))
-    call("loom_paraplex_forward", dtype_code(pc), ptr(pc), ptr(gc), ptr(bc), ptr(bias_c),
-         ptr(trace_c), ptr(tw_c), ptr(rc), ptr(anchor_c),
-         ptr(act), ptr(s), ptr(nxt), ptr(snap), B, T, H, float(m), stream_of(pc))
+    bias_c, trace_c, tw_c, anchor_c = bias.contiguous(), trace.contiguous(), trace_w.contiguous(), anchor.contiguous()
+    call("loom_paraplex_forward", dtype_code(pc), addr(pc), addr(gc), addr(bc), addr(bias_c),
+         addr(trace_c), addr(tw_c), addr(rc), addr(anchor_c),
+         addr(act), addr(s), addr(nxt), addr(snap), B, T, H, float(m), raw_stream(pc.device))
     return [act, s, nxt, snap]
 
 
@@ -105,26 +113,31 @@ def beta_forward_cuda(u, q_h, k_ctx_h, c_h, d_h, w1_imag_compact, hidden_per_q_h
     tile), so ``r_pack`` is an empty tensor; the reference's callers discard it
     (loomformer.py:2497, :2545).
     """
-    ts = (u, q_h, k_ctx_h, c_h, d_h, w1_imag_compact)
-    for nm, t in zip(("u", "q_h", "k_ctx_h", "c_h", "d_h", "w1_imag_compact"), ts):
-        _check(t.is_cuda, f"{nm} must be a CUDA tensor")
-        _check(t.dtype in (torch.float32, torch.bfloat16), f"{nm} must be float32 or bfloat16")
-        _check(t.dtype == u.dtype, f"{nm} dtype mismatch")
-        _check(t.device == u.device, f"{nm} device mismatch")
+    dt, idx = u.dtype, u.get_device()
+    for nm, t in (("u", u), ("q_h", q_h), ("k_ctx_h", k_ctx_h), ("c_h", c_h), ("d_h", d_h),
+                  ("w1_imag_compact", w1_imag_compact)):
+        if not (t.is_cuda and t.dtype == dt and t.get_device() == idx and
+                (dt is torch.bfloat16 or dt is torch.float32)):
+            _check(t.is_cuda, f"{nm} must be a CUDA tensor")
+            _check(t.dtype in (torch.float32, torch.bfloat16), f"{nm} must be float32 or bfloat16")
+            _check(t.dtype == dt, f"{nm} dtype mismatch")
+            _check(t.device == u.device, f"{nm} device mismatch")
     _check(u.dim() == 3, "u must be [B,T,N]")
     B, T, N = u.shape
     H, K = w1_imag_compact.shape
+    sector = (B, T, n_q_heads, head_dim)
     for nm, t in (("q_h", q_h), ("k_ctx_h", k_ctx_h), ("c_h", c_h), ("d_h", d_h)):
-        _check(t.dim() == 4 and tuple(t.shape) == (B, T, n_q_heads, head_dim), f"{nm} must be [B,T,QH,HD]")
+        if t.shape != sector:
+            raise RuntimeError(f"{nm} must be [B,T,QH,HD]")
     _check(N % 4 == 0 and head_dim % 4 == 0 and K % 4 == 0,
            "maskpack path requires N, head_dim, IMAG_IN divisible by 4")
-    out = torch.empty(B, T, H, dtype=u.dtype, device=u.device)
+    out = u.new_empty((B, T, H))
     wc = w1_imag_compact.contiguous()
-    uc, qc, kc, cc, dc = (t.contiguous() for t in (u, q_h, k_ctx_h, c_h, d_h))
-    call("loom_beta_forward", dtype_code(uc), ptr(uc), ptr(qc), ptr(kc), ptr(cc), ptr(dc), ptr(wc),
-         ptr(out), None, B * T, N, H, K, int(hidden_per_q_head), int(head_dim), int(n_q_heads),
-         1 if open_sectors else 0, stream_of(uc))
-    return [out, torch.empty(0, dtype=u.dtype, device=u.device), wc]
+    uc, qc, kc, cc, dc = u.contiguous(), q_h.contiguous(), k_ctx_h.contiguous(), c_h.contiguous(), d_h.contiguous()
+    call("loom_beta_forward", dtype_code(uc), addr(uc), addr(qc), addr(kc), addr(cc), addr(dc), addr(wc),
+         addr(out), None, B * T, N, H, K, int(hidden_per_q_head), int(head_dim), int(n_q_heads),
+         1 if open_sectors else 0, raw_stream(uc.device))
+    return [out, u.new_empty((0,)), wc]
 
 
 def _unsupported(name):
@@ -146,7 +159,7 @@ def phase_sin_forward_cuda(beta: torch.Tensor) -> torch.Tensor:
     _check(beta.dtype in _FLOATS, "phase_sin_forward_cuda: unsupported dtype")
     bc = beta.contiguous()
     out = torch.empty_like(bc)
-    call("loom_phase_sin_forward", dtype_code(bc), ptr(bc), ptr(out), bc.numel(), stream_of(bc))
+    call("loom_phase_sin_forward", dtype_code(bc), addr(bc), addr(out), bc.numel(), raw_stream(bc.device))
     return out
 
 
@@ -161,8 +174,8 @@ def pvpowlu_forward_cuda(x1: torch.Tensor, x2: torch.Tensor, m: float) -> torch.
     _check(x1.dtype == x2.dtype and x1.dtype in _FLOATS, "pvpowlu_forward_cuda: dtype mismatch")
     a, b = x1.contiguous(), x2.contiguous()
     out = torch.empty_like(a)
-    call("loom_pvpowlu_forward", dtype_code(a), ptr(a), ptr(b), ptr(out), a.numel(), float(m),
-         stream_of(a))
+    call("loom_pvpowlu_forward", dtype_code(a), addr(a), addr(b), addr(out), a.numel(), float(m),
+         raw_stream(a.device))
     return out
 
 
@@ -204,8 +217,8 @@ def depth_attn_read(q: torch.Tensor, hist_k: torch.Tensor, hist_v: torch.Tensor,
     d = torch.empty(B, T, QH, HD, dtype=hist_k.dtype, device=hist_k.device)
     w = torch.empty(B, T, QH, S, dtype=hist_k.dtype, device=hist_k.device) if want_weights else None
     lse = torch.empty(B, T, QH, dtype=torch.float32, device=hist_k.device) if want_lse else None
-    call("loom_depth_attn_forward", dtype_code(qc), ptr(qc), ptr(hist_k), ptr(hist_v), sk[0], sk[1],
-         ptr(d), ptr(w), ptr(lse), B * T, S, QH, HD, stream_of(qc))
+    call("loom_depth_attn_forward", dtype_code(qc), addr(qc), addr(hist_k), addr(hist_v), sk[0], sk[1],
+         addr(d), addr(w), addr(lse), B * T, S, QH, HD, raw_stream(qc.device))
     return d, w, lse
 
 
@@ -250,9 +263,9 @@ def _tria_call(r, i, o, prev, seed, valid, w, want_scale, alpha, axis, want_carr
     p = torch.empty_like(rc) if w is not None else None
     scale = torch.empty(n, dtype=torch.float32, device=r.device) if want_scale else None
     prev_c, seed_c, valid_c, w_c = _c(prev), _c(seed), _c(valid), _c(w)
-    call("loom_tria_depth_forward", dtype_code(rc), ptr(rc), ptr(ic), ptr(oc), ptr(prev_c),
-         ptr(seed_c), ptr(valid_c), ptr(w_c), ptr(carry), ptr(p), ptr(scale), B, T, H,
-         float(alpha), int(axis), stream_of(rc))
+    call("loom_tria_depth_forward", dtype_code(rc), addr(rc), addr(ic), addr(oc), addr(prev_c),
+         addr(seed_c), addr(valid_c), addr(w_c), addr(carry), addr(p), addr(scale), B, T, H,
+         float(alpha), int(axis), raw_stream(rc.device))
     return carry, p, scale
 
 
@@ -331,8 +344,8 @@ def gate_slot_mix_forward(carry, w):
     cc = carry.contiguous()
     p = torch.empty(cc.shape[:-2], dtype=cc.dtype, device=cc.device)
     wc = w.contiguous()
-    call("loom_gate_slot_mix_forward", dtype_code(cc), ptr(cc), ptr(wc), ptr(p),
-         cc.numel() // 9, stream_of(cc))
+    call("loom_gate_slot_mix_forward", dtype_code(cc), addr(cc), addr(wc), addr(p),
+         cc.numel() // 9, raw_stream(cc.device))
     return p
 
 
@@ -348,8 +361,8 @@ def slot_attention_pool_forward(carry, score_w):
     pooled = torch.empty(B, T, 9, dtype=cc.dtype, device=cc.device)
     lse = torch.empty(B, T, dtype=cc.dtype, device=cc.device)
     sw = score_w.contiguous()
-    call("loom_slot_attention_pool_forward", dtype_code(cc), ptr(cc), ptr(sw),
-         ptr(pooled), ptr(lse), B * T, H, stream_of(cc))
+    call("loom_slot_attention_pool_forward", dtype_code(cc), addr(cc), addr(sw),
+         addr(pooled), addr(lse), B * T, H, raw_stream(cc.device))
     return [pooled, lse]
 
 
@@ -366,8 +379,8 @@ def temporal_carry_forward(depth_carry, reset_mask):
     doc = torch.empty(dc.shape, dtype=torch.float32, device=dc.device)
     scale = torch.empty(B, T, H, dtype=torch.float32, device=dc.device)
     rm = reset_mask.contiguous()
-    call("loom_temporal_carry_forward", dtype_code(dc), ptr(dc), ptr(rm),
-         ptr(doc), ptr(scale), B, T, H, stream_of(dc))
+    call("loom_temporal_carry_forward", dtype_code(dc), addr(dc), addr(rm),
+         addr(doc), addr(scale), B, T, H, raw_stream(dc.device))
     return [doc, scale]
 
 
@@ -394,8 +407,8 @@ def temporal_carry_endpoint_forward(depth, reset, initial, initial_valid):
     ep = torch.empty(B, H, 3, 3, dtype=dc.dtype, device=dc.device)
     ep32 = torch.empty(B, H, 3, 3, dtype=torch.float32, device=dc.device)
     rs = reset.contiguous()
-    call("loom_temporal_carry_endpoint_forward", dtype_code(dc), ptr(dc), ptr(rs),
-         ptr(init_c), ptr(valid_c), ptr(ep), ptr(ep32), B, T, H, stream_of(dc))
+    call("loom_temporal_carry_endpoint_forward", dtype_code(dc), addr(dc), addr(rs),
+         addr(init_c), addr(valid_c), addr(ep), addr(ep32), B, T, H, raw_stream(dc.device))
     return [ep, ep32]
 
 
@@ -415,8 +428,8 @@ def final_ca_sparse_forward(q, k, v, allowed, scale: float):
     qc, kc, vc, ac = q.contiguous(), k.contiguous(), v.contiguous(), allowed.contiguous()
     out = torch.empty_like(qc)
     lse = torch.empty(B, T, dtype=torch.float32, device=q.device)
-    call("loom_final_ca_sparse_forward", dtype_code(qc), ptr(qc), ptr(kc), ptr(vc),
-         ptr(ac), ptr(out), ptr(lse), B, T, K, D, float(scale), stream_of(qc))
+    call("loom_final_ca_sparse_forward", dtype_code(qc), addr(qc), addr(kc), addr(vc),
+         addr(ac), addr(out), addr(lse), B, T, K, D, float(scale), raw_stream(qc.device))
     return [out, lse]
 
 
@@ -430,8 +443,8 @@ def polarm(matrix: torch.Tensor, beta: float = 0.1, eps: float = 1e-6,
     n = mc.numel() // 9
     per = n // mc.shape[0] if mask is not None else 1
     mk = _c(mask)
-    call("loom_polarm_forward", dtype_code(mc), ptr(mc), ptr(out), ptr(mk), n, per,
-         float(beta), float(eps), stream_of(mc))
+    call("loom_polarm_forward", dtype_code(mc), addr(mc), addr(out), addr(mk), n, per,
+         float(beta), float(eps), raw_stream(mc.device))
     return out
 
 
@@ -469,9 +482,9 @@ def tria_chunked_forward(r: torch.Tensor, i: torch.Tensor, o: torch.Tensor, alph
         keys = torch.empty(B, max(K, 0), H, 3, 3, dtype=torch.float32, device=r.device)
         nbytes = lib.loom_tria_chunked_workspace_bytes(B, T, H, window)
         ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=r.device)
-        call("loom_tria_chunked_forward", dtype_code(rc), ptr(rc), ptr(ic), ptr(oc), B * T * H, L,
-             ptr(rs), ptr(keys) if K > 0 else None, ptr(depth), ptr(ws), nbytes, B, T, H, window,
-             float(alpha), float(polarm_beta), float(eps), stream_of(rc))
+        call("loom_tria_chunked_forward", dtype_code(rc), addr(rc), addr(ic), addr(oc), B * T * H, L,
+             addr(rs), addr(keys) if K > 0 else None, addr(depth), addr(ws), nbytes, B, T, H, window,
+             float(alpha), float(polarm_beta), float(eps), raw_stream(rc.device))
         if not return_valid:
             return keys, depth
         valid = torch.ones(B, max(K, 0), dtype=torch.bool, device=r.device)
@@ -490,10 +503,10 @@ def tria_chunked_forward(r: torch.Tensor, i: torch.Tensor, o: torch.Tensor, alph
     bptr = ctypes.c_void_p(bounds.data_ptr())
     nbytes = lib.loom_tria_chunked_fires_workspace_bytes(B, T, H, bptr, K)
     ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=r.device)
-    call("loom_tria_chunked_forward_fires", dtype_code(rc), ptr(rc), ptr(ic), ptr(oc), B * T * H, L,
-         ptr(rs), ptr(ef), bptr, K, ptr(keys) if K > 0 else None, ptr(kv) if K > 0 else None,
-         ptr(depth), ptr(ws), nbytes, B, T, H, window, float(alpha), float(polarm_beta), float(eps),
-         stream_of(rc))
+    call("loom_tria_chunked_forward_fires", dtype_code(rc), addr(rc), addr(ic), addr(oc), B * T * H, L,
+         addr(rs), addr(ef), bptr, K, addr(keys) if K > 0 else None, addr(kv) if K > 0 else None,
+         addr(depth), addr(ws), nbytes, B, T, H, window, float(alpha), float(polarm_beta), float(eps),
+         raw_stream(rc.device))
     if return_valid:
         return keys, depth, kv.bool()
     return keys, depth
@@ -518,19 +531,26 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     and a residual add.  bias is float32."""
     _check(x.is_cuda and weight.is_cuda, "linear: CUDA tensors required")
     _check(x.dtype == weight.dtype and x.dtype in _FLOATS, "linear: dtype mismatch")
-    K = x.shape[-1]
+    shape = x.shape
+    K = shape[-1]
     _check(weight.dim() == 2 and weight.shape[1] == K, "linear: weight must be [N,K]")
     Nout = weight.shape[0]
-    x2 = x.reshape(-1, K)
-    if x2.stride(-1) != 1:
-        x2 = x2.contiguous()
-    M = x2.shape[0]
+    if K > 0 and x.is_contiguous():
+        x2, ldx = x, K
+        M = x.numel() // K
+    else:
+        x2 = x.reshape(-1, K)
+        if x2.stride(-1) != 1:
+            x2 = x2.contiguous()
+        M, ldx = x2.shape[0], x2.stride(0)
     wc = weight if weight.stride(-1) == 1 else weight.contiguous()
     if out is None:
-        out = torch.empty(*x.shape[:-1], Nout, dtype=x.dtype, device=x.device)
-    b = None if bias is None else bias.float().contiguous()
+        out = x.new_empty((*shape[:-1], Nout))
+    b = bias
+    if b is not None and not (b.dtype is torch.float32 and b.is_contiguous()):
+        b = b.float().contiguous()
     gp = None if gate_p is None else gate_p.reshape(M, Nout).contiguous()
     rs = None if residual is None else residual.reshape(M, Nout).contiguous()
-    call("loom_linear", dtype_code(x2), ptr(x2), x2.stride(0), ptr(wc), wc.stride(0), ptr(b),
-         ptr(gp), float(gate_alpha), ptr(rs), ptr(out), Nout, M, Nout, K, stream_of(x2))
+    call("loom_linear", dtype_code(x2), addr(x2), ldx, addr(wc), wc.stride(0), addr(b),
+         addr(gp), float(gate_alpha), addr(rs), addr(out), Nout, M, Nout, K, raw_stream(x2.device))
     return out

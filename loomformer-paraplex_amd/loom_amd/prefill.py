@@ -26,7 +26,7 @@ import torch
 
 from . import _lib
 
-_P = _lib.ptr
+_P = _lib.addr
 
 # batch rows of a layer's attention on the aux stream (the rest on main, after
 # its depth read): at B = 32, 24 rows measured 62.2-62.3 ms against 62.5-62.6
@@ -62,18 +62,23 @@ def prefill(eng, prompt: torch.Tensor) -> None:
 
 
 def _prefill(eng, prompt: torch.Tensor) -> None:
+    # The host enqueues about 16 launches per layer and chunk; with few rows they
+    # are shorter than it takes to issue them.  So pointers are plain integers
+    # formed from the buffers' addresses (no tensor views), stream handles are
+    # passed to the calls (no stream contexts) and the events are made once: 2 x
+    # 777 tokens through four layers took 7.5 ms, as did 8 x 777.
     c = eng.cfg
     B, P = prompt.shape
     if B != eng.B or P < 1:
         raise ValueError("prompt must be [batch, >=1]")
     eng._check_capacity(P - 1)
-    eng._check_ids(prompt)
+    prompt_cpu = prompt.cpu()
+    eng._check_ids(prompt_cpu)
     N, H, L, QH, KVH, HD = c.N, c.H, c.L, c.QH, c.KVH, c.HD
     dev, dt, code = eng.dev, eng.dtype, eng.code
-    st = eng._stream()
+    lib = eng.lib
     call = eng._call
     prompt_d = prompt.to(dev)
-    prompt_cpu = prompt.cpu()
     ends = chunk_bounds(prompt_cpu, c.window, c.seq_len, eng.carry_token_id)
     hard = torch.tensor([(t + 1) % c.window == 0 and t + 1 < c.seq_len for t in range(P)])
     fire_all = hard[None, :].expand(B, P).clone()
@@ -100,15 +105,10 @@ def _prefill(eng, prompt: torch.Tensor) -> None:
     M = B * Tmax
     h = buf("h", M, N)
     y = buf("y", M, N)
-    qkv = buf("qkv", M, N + 2 * c.KV)
-    q = buf("q", M, QH, HD)
     cbuf = buf("cbuf", M, N)
-    kctx = buf("kctx", M, N)
     d = buf("d", M, N)
     dh = buf("dh", M, N)
     R = buf("R", M, H)
-    gbuf = buf("gbuf", M, H) if c.gate_proj else None
-    beta = buf("beta", M, H)
     act = buf("act", M, H)
     hist = buf("hist", M, 2 * L, 2 * N)
     h0 = buf("h0", M, N)                 # token embeddings of a chunk
@@ -124,87 +124,122 @@ def _prefill(eng, prompt: torch.Tensor) -> None:
     cache_st = HD
     cache_sh = eng.max_len * HD
 
-    def lin(x, w, out, rows, nout, k, **kw):
-        eng._linear(x, w, out, rows, nout, k, **kw)
+    # device addresses
+    E = h.element_size()
+    qkv_p, q_p = buf("qkv", M, N + 2 * c.KV).data_ptr(), buf("q", M, QH, HD).data_ptr()
+    kctx_p, beta_p = buf("kctx", M, N).data_ptr(), buf("beta", M, H).data_ptr()
+    gbuf_p = buf("gbuf", M, H).data_ptr() if c.gate_proj else None
+    h_p, h0_p, c_p, d_p, dh_p = h.data_ptr(), h0.data_ptr(), cbuf.data_ptr(), d.data_ptr(), dh.data_ptr()
+    R_p, act_p, hist_p = R.data_ptr(), act.data_ptr(), hist.data_ptr()
+    state_p, state32_p = state.data_ptr(), state32.data_ptr()
+    carry_p = [carry[i].data_ptr() for i in (0, 1)]
+    pbuf_p = [pbuf[i].data_ptr() for i in (0, 1)]
+    trace_p = [[traces[i, bi].data_ptr() for bi in range(L)] for i in (0, 1)]
+    kc_p = [t.data_ptr() for t in eng.k_cache]
+    vc_p = [t.data_ptr() for t in eng.v_cache]
+    qp_p = [t.data_ptr() for t in eng.qp]
+    kvw_p, cos_p, sin_p = eng.kvw.data_ptr(), eng.cos.data_ptr(), eng.sin.data_ptr()
+    slot = 2 * N * E                     # bytes of one history slot of a row
+    hist_ld = 2 * L * 2 * N              # elements between rows of a history slot
 
     # LayerNorm(x w^T + x2 w2^T + bias) -> h (y: the product, on the unfused path)
-    ln_ws = buf("ln_ws", _lib.load().loom_linear_ln_workspace_bytes(M, N) // 4, dtype=torch.float32)
+    ln_ws = buf("ln_ws", lib.loom_linear_ln_workspace_bytes(M, N) // 4, dtype=torch.float32)
+    ln_p, ln_bytes = ln_ws.data_ptr(), ln_ws.numel() * 4
+
+    main = torch.cuda.current_stream(dev)
+    aux = eng.aux_stream
+    tail = eng.tail_stream        # a chunk's temporal carry and document key
+    st, aux_st, tail_st = main.cuda_stream, aux.cuda_stream, tail.cuda_stream
 
     descs = {}
 
     def lin_ln(key, x, w, x2, w2, bias, gamma, beta_ln, rows):
         dsc = descs.get((key, rows))
         if dsc is None:
-            dsc = descs[(key, rows)] = _lib.linear_multi_desc(
-                x[:rows], [dict(w=w, w2=w2, out=y[:rows], bias=bias)], x2=x2[:rows])
-        call("loom_linear_ln", code, _lib.ctypes.byref(dsc), _P(gamma), _P(beta_ln), 1e-5, _P(h), N,
-             _P(ln_ws), ln_ws.numel() * 4, None, st)
+            dd = _lib.linear_multi_desc(x[:rows], [dict(w=w, w2=w2, out=y[:rows], bias=bias)], x2=x2[:rows])
+            dsc = descs[(key, rows)] = (dd, _lib.ctypes.byref(dd), gamma.data_ptr(), beta_ln.data_ptr())
+        call("loom_linear_ln", code, dsc[1], dsc[2], dsc[3], 1e-5, h_p, N, ln_p, ln_bytes, None, st)
 
     # the attention sublayer's read of slots 0..2bi also reads them with the FFN
     # sublayer's query (its part, fp32); the FFN read then folds in slot 2bi+1
     pair = eng.pair_reads
-    part_d = buf("part_d", M, QH, HD, dtype=torch.float32) if pair else None
-    part_lse = buf("part_lse", M, QH, dtype=torch.float32) if pair else None
+    if pair:
+        part_d_p = buf("part_d", M, QH, HD, dtype=torch.float32).data_ptr()
+        part_lse_p = buf("part_lse", M, QH, dtype=torch.float32).data_ptr()
 
-    def depth(sub, out, rows):
+    def depth(sub, out_p, rows):
+        """DepthAttn read of sublayer sub over slots [0, sub] (loomformer.py:3404-3429)
+        on main: one pass over slots [0, sub] for sublayers sub and sub + 1 (the
+        latter's part over them in fp32), then the fold of the last slot."""
         if not pair:
-            eng.depth_read(sub, hist, out, rows)
+            if eng.depth_rms is None:
+                call("loom_depth_attn_forward", code, qp_p[sub], hist_p, hist_p + N * E, hist_ld, 2 * N, out_p, None,
+                     None, rows, sub + 1, QH, HD, st)
+            else:
+                call("loom_depth_attn_forward_rms", code, qp_p[sub], hist_p, hist_p + N * E, hist_ld, 2 * N, out_p,
+                     None, None, rows, sub + 1, QH, HD, *eng.depth_rms, st)
         elif sub % 2 == 0:
-            eng.depth_read_pair(sub, hist, out, part_d, part_lse, rows)
+            call("loom_depth_attn_pair", code, qp_p[sub], qp_p[sub + 1], hist_p, hist_p + N * E, hist_ld, 2 * N,
+                 out_p, part_d_p, part_lse_p, rows, sub + 1, QH, HD, st)
         else:
-            eng.depth_read_fold(sub, hist, out, part_d, part_lse, rows)
+            call("loom_depth_attn_fold", code, qp_p[sub], hist_p, hist_p + N * E, hist_ld, 2 * N, sub + 1, part_d_p,
+                 part_lse_p, out_p, rows, QH, HD, st)
 
     spans = list(zip([0] + [x + 1 for x in ends[:-1]], ends))
 
+    # each event is recorded again and again: a wait takes the record before it
     gathered = torch.cuda.Event()
     qkv_ready = torch.cuda.Event()      # a layer's q and cache rows written (aux)
+    forked, joined = torch.cuda.Event(), torch.cuda.Event()
     # batch rows whose attention runs on aux right after the qkv product; the
     # rest run on main after its depth read (the two branches then take about
     # as long)
     aux_rows = min(B, PREFILL_AUX_ROWS)
 
-    def next_qkv(x, bi, sub, s_, Tc_):
+    def next_qkv(x_p, bi, sub, s_, Tc_):
         """Block bi's qkv of x with RoPE + cache append (loomformer.py:3262, :3300-3320)
         and, unless sub is None, history slot `sub` (DepthAttn.project, :3397): one
-        launch where the shapes allow, on the current stream; the attention then runs
-        with qkv = NULL."""
-        wh = None if sub is None else _P(eng.kvw)
-        ho = None if sub is None else _P(hist[:, sub])
-        call("loom_prefill_qkv", code, _P(x), N, _P(eng.blocks[bi]["qkv"]), wh, ho, 2 * L * 2 * N,
-             2 * N, _P(qkv), _P(q), _P(eng.k_cache[bi]), _P(eng.v_cache[bi]), cache_sb, cache_st,
-             cache_sh, _P(eng.cos), _P(eng.sin), B, Tc_, s_, eng.max_len, N, QH, KVH, HD,
-             eng._stream())
+        launch where the shapes allow, on aux; the attention then runs with
+        qkv = NULL."""
+        call("loom_prefill_qkv", code, x_p, N, blocks[bi]["qkv"], None if sub is None else kvw_p,
+             None if sub is None else hist_p + sub * slot, hist_ld, 2 * N, qkv_p, q_p, kc_p[bi], vc_p[bi],
+             cache_sb, cache_st, cache_sh, cos_p, sin_p, B, Tc_, s_, eng.max_len, N, QH, KVH, HD, aux_st)
 
-    def attend(bi, s_, Tc_, b0=0, b1=B):
+    def attend(bi, s_, Tc_, b0, b1, stream):
         """Block bi's attention for batch rows b0..b1-1 (their cache rows and
-        chunk rows are contiguous views), on the current stream."""
-        r0 = b0 * Tc_
-        call("loom_gqa_prefill", code, None, 0, _P(eng.k_cache[bi][b0:]), _P(eng.v_cache[bi][b0:]),
-             cache_sb, cache_st, cache_sh, _P(eng.cos), _P(eng.sin), _P(q[r0:]), _P(cbuf[r0:]),
-             _P(kctx[r0:]), N, b1 - b0, Tc_, s_, eng.max_len, QH, KVH, HD, eng._stream())
+        chunk rows are contiguous views)."""
+        r0 = b0 * Tc_ * N * E
+        k0 = b0 * cache_sb * E
+        call("loom_gqa_prefill", code, None, 0, kc_p[bi] + k0, vc_p[bi] + k0, cache_sb, cache_st, cache_sh, cos_p,
+             sin_p, q_p + r0, c_p + r0, kctx_p + r0, N, b1 - b0, Tc_, s_, eng.max_len, QH, KVH, HD, stream)
 
     def chunk_head(ci):
         """Layer 0's attention inputs of chunk ci, which need only the chunk's
         tokens and the layer-0 K/V rows of earlier chunks: embeddings, qkv with
-        RoPE + cache append and history slot 0, attention (on the current stream;
-        `gathered` is recorded once history slot 0 is written)."""
+        RoPE + cache append and history slot 0, attention (on aux; `gathered` is
+        recorded once history slot 0 is written)."""
         s_, e_ = spans[ci]
         rows_ = B * (e_ - s_ + 1)
-        torch.index_select(eng.emb, 0, prompt_d[:, s_:e_ + 1].reshape(-1), out=h0[:rows_])
-        next_qkv(h0, 0, 0, s_, e_ - s_ + 1)
-        gathered.record()
-        attend(0, s_, e_ - s_ + 1)
+        with torch.cuda.stream(aux):
+            torch.index_select(eng.emb, 0, prompt_d[:, s_:e_ + 1].reshape(-1), out=h0[:rows_])
+        next_qkv(h0_p, 0, 0, s_, e_ - s_ + 1)
+        gathered.record(aux)
+        attend(0, s_, e_ - s_ + 1, 0, B, aux_st)
 
-    main = torch.cuda.current_stream(dev)
-    aux = eng.aux_stream
-    tail = eng.tail_stream        # a chunk's temporal carry and document key
-    tail_st = _lib.c_void_p(tail.cuda_stream)
+    # the blocks' parameters as addresses (tensors where a descriptor takes them)
+    blocks = [{k: (v.data_ptr() if k in ("qkv", "w1i", "ib", "tw", "gate_w", "gpw", "gpb") else v)
+               for k, v in blk.items()} for blk in eng.blocks]
+
+    def lin(x, w, out, rows, nout, k, **kw):
+        eng._linear(x, w, out, rows, nout, k, **kw)
 
     def fork():                 # aux continues after everything queued on main so far
-        aux.wait_stream(main)
+        forked.record(main)
+        aux.wait_event(forked)
 
     def join():                 # main continues after everything queued on aux so far
-        main.wait_stream(aux)
+        joined.record(aux)
+        main.wait_event(joined)
 
     have_state = False
     tin = 0
@@ -218,8 +253,7 @@ def _prefill(eng, prompt: torch.Tensor) -> None:
     # FFN tail), and `tail` takes the chunk's temporal carry and document key
     # beside the next chunk's first sublayer.
     fork()
-    with torch.cuda.stream(aux):
-        chunk_head(0)
+    chunk_head(0)
     for ci, (s, e) in enumerate(spans):
         Tc = e - s + 1
         rows = B * Tc
@@ -227,22 +261,21 @@ def _prefill(eng, prompt: torch.Tensor) -> None:
         sub = 0
         # the depth read of history slot 0, on main once the slot is written
         main.wait_event(gathered)
-        depth(0, d, rows)
+        depth(0, d_p, rows)
         carry_i, p_i = None, None
-        for bi, blk in enumerate(eng.blocks):
+        for bi, blk in enumerate(blocks):
             last = bi == L - 1
             # ---- attention over the cache (rows < s) and this chunk (loomformer.py:3215-3332),
             # on aux after this layer's qkv; the depth read 2*bi on main (layer 0's
             # ran ahead on aux)
             if bi > 0:
-                with torch.cuda.stream(aux):
-                    attend(bi, s, Tc, 0, aux_rows)
-                depth(sub, d, rows)
+                attend(bi, s, Tc, 0, aux_rows, aux_st)
+                depth(sub, d_p, rows)
                 if aux_rows < B:
                     # the other rows' attention on main after its depth read,
                     # once aux has written this layer's q and cache rows
                     main.wait_event(qkv_ready)
-                    attend(bi, s, Tc, aux_rows, B)
+                    attend(bi, s, Tc, aux_rows, B, st)
             join()
             # ---- LN(o(C) + w_o(depth read 2*bi)) (loomformer.py:3999-4000)
             lin_ln(("attn", bi), cbuf, blk["o"], d, eng.wo_for(sub), None, blk["ln1_w"], blk["ln1_b"],
@@ -258,26 +291,24 @@ def _prefill(eng, prompt: torch.Tensor) -> None:
                 real = dict(w=blk["w1r"], out=R[:rows], bias=blk["b1r"])
                 if p_i is not None:
                     real.update(gate_p=pbuf[p_i][:rows], gate_alpha=blk["alpha"])
-                dsc = descs[key] = _lib.linear_multi_desc(h[:rows], [real, dict(w=eng.kvw, out=hv[:, sub])])
-            call("loom_linear_multi", code, _lib.ctypes.byref(dsc), st)
-            depth(sub, dh, rows)
+                dd = _lib.linear_multi_desc(h[:rows], [real, dict(w=eng.kvw, out=hv[:, sub])])
+                dsc = descs[key] = (dd, _lib.ctypes.byref(dd))
+            call("loom_linear_multi", code, dsc[1], st)
+            depth(sub, dh_p, rows)
             # ---- Paraplex FFN (loomformer.py:2818-2893): beta space, fused pointwise
             # chain with the phase trace carried from the previous chunk; the
             # amplitude source is R, or gate_proj(h) under paraplex_gate_proj (:2849)
-            call("loom_beta_forward", code, _P(h), _P(q), _P(kctx), _P(cbuf), _P(dh),
-                 _P(blk["w1i"]), _P(beta), None, rows, N, H, c.imag_in, c.Hq, HD, QH,
-                 1 if c.sectors == "open" else 0, st)
-            gsrc = R
+            call("loom_beta_forward", code, h_p, q_p, kctx_p, c_p, dh_p, blk["w1i"], beta_p, None, rows, N, H,
+                 c.imag_in, c.Hq, HD, QH, 1 if c.sectors == "open" else 0, st)
+            gsrc_p = R_p
             if c.gate_proj:
-                gsrc = gbuf
-                lin(h, blk["gpw"], gbuf, rows, H, N, bias=blk["gpb"])
-            join()
+                gsrc_p = gbuf_p
+                call("loom_linear", code, h_p, N, blk["gpw"], N, blk["gpb"], None, 0.0, None, gbuf_p, H, rows, H, N, st)
             if last and ci + 1 < len(spans):
                 # the next chunk's layer-0 attention inputs, after this layer's
                 # beta space has read q, kctx and c
                 fork()
-                with torch.cuda.stream(aux):
-                    chunk_head(ci + 1)
+                chunk_head(ci + 1)
             # ---- with the block's Tria depth op (loomformer.py:3588-3617), axis bi % 3,
             # in the same pass: the phase I never leaves the chip
             out_i = 0 if carry_i != 0 else 1
@@ -296,20 +327,16 @@ def _prefill(eng, prompt: torch.Tensor) -> None:
                     reset[:, 0] = 1
                 else:
                     reset[:, 0] = seed_valid
-                call("loom_paraplex_tria_endpoint_forward", code, _P(R), _P(gsrc), _P(beta),
-                     _P(blk["ib"]), _P(traces[tin, bi]), _P(blk["tw"]), float(c.powlu_m),
-                     _P(carry[carry_i]), _P(reset), _P(state) if have_state else None, None,
-                     _P(act), _P(traces[1 - tin, bi]), _P(state), _P(state32), B, Tc, H,
-                     float(c.tria_alpha), bi % 3, st)
+                call("loom_paraplex_tria_endpoint_forward", code, R_p, gsrc_p, beta_p, blk["ib"], trace_p[tin][bi],
+                     blk["tw"], c.powlu_m, carry_p[carry_i], reset.data_ptr(), state_p if have_state else None, None,
+                     act_p, trace_p[1 - tin][bi], state_p, state32_p, B, Tc, H, c.tria_alpha, bi % 3, st)
                 endpoint_done = True
             else:
-                call("loom_paraplex_tria_forward", code, _P(R), _P(gsrc), _P(beta), _P(blk["ib"]),
-                     _P(traces[tin, bi]), _P(blk["tw"]), float(c.powlu_m),
-                     None if (carry_i is None or seeded) else _P(carry[carry_i]),
-                     _P(state) if seeded else None, _P(seed_valid) if seeded else None,
-                     _P(blk["gate_w"]) if gate else None, _P(act), _P(traces[1 - tin, bi]),
-                     _P(carry[out_i]), _P(pbuf[new_p]) if gate else None, B, Tc, H,
-                     float(c.tria_alpha), bi % 3, st)
+                call("loom_paraplex_tria_forward", code, R_p, gsrc_p, beta_p, blk["ib"], trace_p[tin][bi], blk["tw"],
+                     c.powlu_m, None if (carry_i is None or seeded) else carry_p[carry_i],
+                     state_p if seeded else None, seed_valid.data_ptr() if seeded else None,
+                     blk["gate_w"] if gate else None, act_p, trace_p[1 - tin][bi], carry_p[out_i],
+                     pbuf_p[new_p] if gate else None, B, Tc, H, c.tria_alpha, bi % 3, st)
                 endpoint_done = False
             carry_i, p_i = out_i, new_p
             if last:
@@ -322,10 +349,10 @@ def _prefill(eng, prompt: torch.Tensor) -> None:
                 # qkv with RoPE + cache append on aux (its attention follows there)
                 sub += 1
                 fork()
-                with torch.cuda.stream(aux):
-                    next_qkv(h, bi + 1, None, s, Tc)
-                    qkv_ready.record()
-                lin(h, eng.kvw, hv[:, sub], rows, 2 * N, N, ldc=2 * L * 2 * N)
+                next_qkv(h_p, bi + 1, None, s, Tc)
+                qkv_ready.record(aux)
+                call("loom_linear", code, h_p, N, kvw_p, N, None, None, 0.0, None, hist_p + sub * slot, hist_ld, rows,
+                     2 * N, N, st)
         # ---- on the third stream, beside the next chunk's first sublayer: the
         # temporal carry over the chunk, restarting at position 0 and at a
         # seeded first token, else continuing from the state (loomformer.py:3834-3850)
@@ -336,9 +363,8 @@ def _prefill(eng, prompt: torch.Tensor) -> None:
                     reset[:, 0] = 1
                 else:
                     reset[:, 0] = seed_valid
-                call("loom_temporal_carry_endpoint_forward", code, _P(carry[carry_i]), _P(reset),
-                     _P(state) if have_state else None, None, _P(state), _P(state32), B, Tc, H,
-                     tail_st)
+                call("loom_temporal_carry_endpoint_forward", code, carry_p[carry_i], _P(reset),
+                     state_p if have_state else None, None, state_p, state32_p, B, Tc, H, tail_st)
             have_state = True
             fire_e = fire_all_d[:, e]
             if bool(fire_all[:, e].any()):
