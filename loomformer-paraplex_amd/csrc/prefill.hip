@@ -310,8 +310,14 @@ constexpr int kPfRows = 32 * kPfSub;   // cached rows per step
 // accumulators sit in ordinary VGPRs, where the per-step rescale multiplies
 // them in place (in AGPRs each would be copied out and back, 144 VALU
 // operations per step)
-template <int HD, int GP, int HSPLIT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+//
+// KS = 2: eight waves, two groups of four that take alternate 64-row steps of
+// the same queries (each its own LDS stages) and are merged at the end, for
+// grids that give a CU one block at most: half the steps in sequence.  The
+// second group may see no row of an early query, so the running maximum starts
+// at a finite floor instead of -inf there.
+template <int HD, int GP, int HSPLIT, int KS>
+__global__ void __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 gqa_prefill_mfma_kernel(PrefillArgs<bf16_t> a) {
     constexpr int KK = HD / 32;
     constexpr int DT = HD / 16;
@@ -325,18 +331,20 @@ gqa_prefill_mfma_kernel(PrefillArgs<bf16_t> a) {
     // (tile t in stage t % 3) as separate arrays, so that a wait for one
     // stage's loads never covers another stage's reads
     constexpr int PITCH = CPR;
-    __shared__ __align__(16) gqa_u4 K0[R * PITCH], K1[R * PITCH], K2[R * PITCH];
-    __shared__ __align__(16) gqa_u4 V0[R * PITCH], V1[R * PITCH], V2[R * PITCH];
-    __shared__ float cr[4][16];                           // per-column rescale of a step
+    __shared__ __align__(16) gqa_u4 K0[KS * R * PITCH], K1[KS * R * PITCH], K2[KS * R * PITCH];
+    __shared__ __align__(16) gqa_u4 V0[KS * R * PITCH], V1[KS * R * PITCH], V2[KS * R * PITCH];
+    __shared__ float cr[4 * KS][16];                      // per-column rescale of a step
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = KS == 1 ? tid >> 6 : wave8 & 3, grp = KS == 1 ? 0 : wave8 >> 2;
     auto kst = [&](auto s_) -> gqa_u4* {
         constexpr int S = decltype(s_)::value;
-        return S == 0 ? K0 : S == 1 ? K1 : K2;
+        return (S == 0 ? K0 : S == 1 ? K1 : K2) + grp * R * PITCH;
     };
     auto vst = [&](auto s_) -> gqa_u4* {
         constexpr int S = decltype(s_)::value;
-        return S == 0 ? V0 : S == 1 ? V1 : V2;
+        return (S == 0 ? V0 : S == 1 ? V1 : V2) + grp * R * PITCH;
     };
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int lr = lane & 15, lq = lane >> 4;
     // work item (query tiles, head group, row) in query-tile-fastest order; the
     // query tiles of one (row, kv head) read the same K/V rows, so they share
@@ -349,7 +357,7 @@ gqa_prefill_mfma_kernel(PrefillArgs<bf16_t> a) {
     const int head = kvh * G + part * GP + wave % GP;
     const int qlast_blk = min((bx + 1) * QTB * 16, a.Tc) - 1;
     const int64_t kmax = a.start + qlast_blk;                    // last cached row the block reads
-    const int nsteps = (int)((kmax + R) / R);
+    const int nsteps = (int)((kmax + KS * R) / (KS * R));        // per group
     const int q0 = (bx * QTB + wave / GP) * 16;                  // first query of the wave's tile
     // this lane's query column (lr): its position; a column past the chunk
     // attends to row 0 only (finite, never stored)
@@ -402,14 +410,14 @@ gqa_prefill_mfma_kernel(PrefillArgs<bf16_t> a) {
         for (int kk = 0; kk < KK; ++kk)
             qf[kk] = *reinterpret_cast<const uint4*>(qp + 32 * kk + 8 * lq);
     }
-    load_tile(S0{}, 0);
-    load_tile(S1{}, R);
+    load_tile(S0{}, grp * R);
+    load_tile(S1{}, (KS + grp) * R);
     dma_barrier<2 * GPW>();                 // q and tile 0 (tile 1 may be in flight)
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk)
         asm volatile("" : "+v"(qf[kk].x), "+v"(qf[kk].y), "+v"(qf[kk].z), "+v"(qf[kk].w));
 
-    float mh = -INFINITY, lh = 0.0f;      // running max / sum of query column lr
+    float mh = KS == 1 ? -INFINITY : -3.0e38f, lh = 0.0f;      // running max / sum of query column lr
     f32x4_p accC[DT], accK[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) accC[dt] = accK[dt] = f32x4_p{0.f, 0.f, 0.f, 0.f};
@@ -424,8 +432,8 @@ gqa_prefill_mfma_kernel(PrefillArgs<bf16_t> a) {
         constexpr int cur = decltype(s_)::value;
         const gqa_u4* tk = kst(s_);
         const gqa_u4* tv = vst(s_);
-        const int64_t r0 = (int64_t)it * R;
-        load_tile(std::integral_constant<int, (cur + 2) % 3>{}, r0 + 2 * R);
+        const int64_t r0 = (int64_t)(KS * it + grp) * R;
+        load_tile(std::integral_constant<int, (cur + 2) % 3>{}, r0 + 2 * KS * R);
         const bool active = r0 <= wave_kmax;                 // wave-uniform
         if (active) {
             // sub-tile u: rows 32u .. 32u + 31 of the step (tile rows from 32u on);
@@ -470,7 +478,7 @@ gqa_prefill_mfma_kernel(PrefillArgs<bf16_t> a) {
             }
             mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            const float mnew = fmaxf(mh, mx * a.qscale);    // finite: row 0 is seen at step 0
+            const float mnew = fmaxf(mh, mx * a.qscale);    // finite: row 0 is seen at step 0 (or the floor)
             const float corr = __builtin_amdgcn_exp2f(mh - mnew);
             float ls = 0.0f, pv[SUB][2][4];
 #pragma unroll
@@ -500,11 +508,11 @@ gqa_prefill_mfma_kernel(PrefillArgs<bf16_t> a) {
             // faster here than four cross-lane permutes); skipped when no
             // column's max moved (every factor exactly 1)
             if (__any(corr != 1.0f)) {
-                if (lq == 0) cr[wave][lr] = corr;
+                if (lq == 0) cr[4 * grp + wave][lr] = corr;
                 wave_lds_fence();
                 float cf[4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) cf[r] = cr[wave][4 * lq + r];
+                for (int r = 0; r < 4; ++r) cf[r] = cr[4 * grp + wave][4 * lq + r];
 #pragma unroll
                 for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -531,6 +539,40 @@ gqa_prefill_mfma_kernel(PrefillArgs<bf16_t> a) {
         step(S2{}, it + 2);
     }
     wait_vmcnt<0>();                        // no load into LDS outlives the loop
+    if constexpr (KS == 2) {
+        // the second group's state through the freed stages (wave w's 64 lanes of
+        // fp32x4, its maxima and sums after them), merged by the first
+        __syncthreads();
+        f32x4_p* const st = reinterpret_cast<f32x4_p*>(K0);
+        f32x4_p* const sv = reinterpret_cast<f32x4_p*>(V0);
+        float* const sm = reinterpret_cast<float*>(K1);
+        static_assert(DT * 256 * 16 <= KS * R * PITCH * 16 && 512 * 4 <= KS * R * PITCH * 16, "merge buffers");
+        if (grp == 1) {
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) {
+                st[(dt * 4 + wave) * 64 + lane] = accC[dt];
+                sv[(dt * 4 + wave) * 64 + lane] = accK[dt];
+            }
+            sm[wave * 64 + lane] = mh;
+            sm[256 + wave * 64 + lane] = lh;
+        }
+        __syncthreads();
+        if (grp == 1) return;
+        const float m1 = sm[wave * 64 + lane], l1 = sm[256 + wave * 64 + lane];
+        const float mm = fmaxf(mh, m1);                  // finite: this group saw row 0
+        const float w0 = __builtin_amdgcn_exp2f(mh - mm), w1 = __builtin_amdgcn_exp2f(m1 - mm);
+        lh = fmaf(lh, w0, l1 * w1);
+        // the factors of the query columns 4*lq + r this lane accumulates
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float f0 = __shfl(w0, 4 * lq + r, 64), f1 = __shfl(w1, 4 * lq + r, 64);
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) {
+                accC[dt][r] = fmaf(accC[dt][r], f0, st[(dt * 4 + wave) * 64 + lane][r] * f1);
+                accK[dt][r] = fmaf(accK[dt][r], f0, sv[(dt * 4 + wave) * 64 + lane][r] * f1);
+            }
+        }
+    }
     // normalise: the sum of query column c lives in lanes with lr == c
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -621,30 +663,41 @@ static int prefill_dispatch(const void* qkv, int64_t qkv_ld, void* kc, void* vc,
     const int G = (int)(QH / KVH);
     if constexpr (std::is_same<T, bf16_t>::value) {
         // the MFMA form addresses a (row, kv head)'s cache rows with 32-bit
-        // byte offsets, up to four tiles past the chunk's last position
+        // byte offsets, up to twelve tiles past the chunk's last position
         const bool mf_ok = (HD == 32 || HD == 64 || HD == 96 || HD == 128) &&
                            (G == 1 || G == 2 || G == 4 || G == 8) &&
-                           (start + Tc + 4 * kPfRows) * cst * 2 < ((int64_t)1 << 31);
+                           (start + Tc + 12 * kPfRows) * cst * 2 < ((int64_t)1 << 31);
         if (mf_ok) {
+            // blocks: 4 (query tile, head) pairs each; two key groups per block where a
+            // CU has no more than one block and there are four steps to share (with
+            // RoPE + append, us: 8 x 128 queries over 1152 rows 27.2 -> 23.8, 1 x 128
+            // 25.4 -> 21.7, 16 x 128 over 640 21.4 -> 20.4; 4 x 128 over 138 10.8 -> 11.5).
+            // HD 128's stages fill the LDS with one group.
+            const int64_t per = G == 4 ? 16 : G == 8 ? 16 : G == 2 ? 32 : 64;
+            const int64_t blocks = ceil_div(Tc, per) * KVH * B * (G == 8 ? 2 : 1);
+            const bool two = HD < 128 && blocks <= (int64_t)device_cus() && start + Tc > 3 * kPfRows;
+            const dim3 g((unsigned)blocks);
+#define LOOM_PF_GO(HDV, GP, HS)                                                                  \
+            do {                                                                                 \
+                if constexpr (HDV < 128) {                                                       \
+                    if (two) {                                                                   \
+                        hipLaunchKernelGGL((gqa_prefill_mfma_kernel<HDV, GP, HS, 2>), g, dim3(512), 0, st, a); \
+                        break;                                                                   \
+                    }                                                                            \
+                }                                                                                \
+                hipLaunchKernelGGL((gqa_prefill_mfma_kernel<HDV, GP, HS, 1>), g, dim3(256), 0, st, a); \
+            } while (0)
 #define LOOM_PF_MF(HDV)                                                                          \
             if (HD == HDV) {                                                                     \
-                if (G == 4) {                                                                    \
-                    const dim3 g((unsigned)(ceil_div(Tc, 16) * KVH * B));                \
-                    hipLaunchKernelGGL((gqa_prefill_mfma_kernel<HDV, 4, 1>), g, dim3(256), 0, st, a); \
-                } else if (G == 8) {                                                             \
-                    const dim3 g((unsigned)(ceil_div(Tc, 16) * KVH * 2 * B));            \
-                    hipLaunchKernelGGL((gqa_prefill_mfma_kernel<HDV, 4, 2>), g, dim3(256), 0, st, a); \
-                } else if (G == 2) {                                                             \
-                    const dim3 g((unsigned)(ceil_div(Tc, 32) * KVH * B));                \
-                    hipLaunchKernelGGL((gqa_prefill_mfma_kernel<HDV, 2, 1>), g, dim3(256), 0, st, a); \
-                } else {                                                                         \
-                    const dim3 g((unsigned)(ceil_div(Tc, 64) * KVH * B));                \
-                    hipLaunchKernelGGL((gqa_prefill_mfma_kernel<HDV, 1, 1>), g, dim3(256), 0, st, a); \
-                }                                                                                \
+                if (G == 4) LOOM_PF_GO(HDV, 4, 1);                                               \
+                else if (G == 8) LOOM_PF_GO(HDV, 4, 2);                                          \
+                else if (G == 2) LOOM_PF_GO(HDV, 2, 1);                                          \
+                else LOOM_PF_GO(HDV, 1, 1);                                                      \
                 return launch_status("loom_gqa_prefill");                                       \
             }
             LOOM_PF_MF(96) LOOM_PF_MF(64) LOOM_PF_MF(128) LOOM_PF_MF(32)
 #undef LOOM_PF_MF
+#undef LOOM_PF_GO
         }
     }
     dim3 grid((unsigned)Tc, (unsigned)KVH, (unsigned)B);
