@@ -1098,7 +1098,7 @@ __device__ __forceinline__ void ffn_tria(const FfnArgs& f, int64_t e, float r, f
 #pragma unroll
         for (int k = 0; k < 9; ++k) pre[k] = mt[k];
     }
-    const float inv = 1.0f / rms9(pre);
+    const float inv = rms9_inv(pre);
 #pragma unroll
     for (int k = 0; k < 9; ++k) pre[k] *= inv;
     if (f.gate_w != nullptr) {

@@ -6,16 +6,23 @@
 
 namespace loom {
 
-// Local carrier T(r,i,o) = (I + K(a,b,c)) @ R_axis,
-// (a,b,c) = alpha * tanh(x / sqrt(mean(x^2) + eps)), x = (ri, ro, io).
-// The axis is a compile-time parameter: the kernels are instantiated per axis.
+// tanh(y) for |y| <= sqrt(3) as y N(y^2) / D(y^2), fitted to a relative error
+// of 5e-9 there (least squares on the relative error over Chebyshev points);
+// with rounding and v_rcp_f32 it stays within 2.4e-7 relative.  Fourteen
+// operations without a branch, where libm's tanhf with the IEEE square root and
+// division around it took most of the element-wise kernels' VALU work; the
+// form 1 - 2 / (1 + e^2y) loses the low bits of small y.
+__device__ __forceinline__ float tanh_unit(float y) {
+    const float z = y * y;
+    const float n = fmaf(z, fmaf(z, 0.0019643290f, 0.1206163f), 1.0f);
+    const float d = fmaf(z, fmaf(z, fmaf(z, 9.0792593e-5f, 0.019947553f), 0.45394963f), 1.0f);
+    return y * n * __builtin_amdgcn_rcpf(d);
+}
+
+// The carrier's rows from (a, b, c); the axis is a compile-time parameter: the
+// kernels are instantiated per axis.
 template <int AXIS>
-__device__ __forceinline__ void carrier9(float r, float i, float o, float alpha, float mt[9]) {
-    const float x0 = r * i, x1 = r * o, x2 = i * o;
-    const float inv = 1.0f / sqrtf((x0 * x0 + x1 * x1 + x2 * x2) * (1.0f / 3.0f) + 1e-6f);
-    const float a = alpha * tanhf(x0 * inv);
-    const float b = alpha * tanhf(x1 * inv);
-    const float c = alpha * tanhf(x2 * inv);
+__device__ __forceinline__ void carrier_rows(float a, float b, float c, float mt[9]) {
     if constexpr (AXIS == 0) {          // about z
         mt[0] = -c;   mt[1] = -1.0f; mt[2] = b;
         mt[3] = 1.0f; mt[4] = -c;    mt[5] = -a;
@@ -31,12 +38,23 @@ __device__ __forceinline__ void carrier9(float r, float i, float o, float alpha,
     }
 }
 
-// carrier9 with the hardware transcendentals, for the streaming chains where
-// the libm forms dominate the instruction count:
-//   1/sqrt -> v_rsq_f32, and tanh(y) = 1 - 2/(1 + 2^(2 y log2 e)) with v_exp_f32
-//   and v_rcp_f32 (1 ulp each).  The tanh argument is x/rms(x), |y| <= sqrt(3),
-//   so the exponential stays in range and the absolute error of alpha*tanh is
-//   a few ulp of alpha.
+// Local carrier T(r,i,o) = (I + K(a,b,c)) @ R_axis,
+// (a,b,c) = alpha * tanh(x / sqrt(mean(x^2) + eps)), x = (ri, ro, io).
+// 1/sqrt is v_rsq_f32 (1 ulp), so |y| <= sqrt(3) and tanh is tanh_unit.
+template <int AXIS>
+__device__ __forceinline__ void carrier9(float r, float i, float o, float alpha, float mt[9]) {
+    const float x0 = r * i, x1 = r * o, x2 = i * o;
+    const float inv = __builtin_amdgcn_rsqf(
+        fmaf(fmaf(x0, x0, fmaf(x1, x1, x2 * x2)), 1.0f / 3.0f, 1e-6f));
+    carrier_rows<AXIS>(alpha * tanh_unit(x0 * inv), alpha * tanh_unit(x1 * inv),
+                       alpha * tanh_unit(x2 * inv), mt);
+}
+
+// carrier9 with tanh(y) = 1 - 2/(1 + 2^(2 y log2 e)) on v_exp_f32 and v_rcp_f32
+// (1 ulp each), for the streaming chains, which the vector ALU bounds (the
+// other form there: 5.63 ms against 4.93 at 24 layers of 8 x 4096 x 3072).  |y| <= sqrt(3),
+// so the exponential stays in range and the absolute error of alpha*tanh is a
+// few ulp of alpha.
 template <int AXIS>
 __device__ __forceinline__ void carrier9_fast(float r, float i, float o, float alpha,
                                               float mt[9]) {
@@ -48,28 +66,27 @@ __device__ __forceinline__ void carrier9_fast(float r, float i, float o, float a
     const float a = fmaf(m2a, __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x0 * k)), alpha);
     const float b = fmaf(m2a, __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x1 * k)), alpha);
     const float c = fmaf(m2a, __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x2 * k)), alpha);
-    if constexpr (AXIS == 0) {
-        mt[0] = -c;   mt[1] = -1.0f; mt[2] = b;
-        mt[3] = 1.0f; mt[4] = -c;    mt[5] = -a;
-        mt[6] = a;    mt[7] = b;     mt[8] = 1.0f;
-    } else if constexpr (AXIS == 1) {
-        mt[0] = 1.0f; mt[1] = b;     mt[2] = c;
-        mt[3] = c;    mt[4] = -a;    mt[5] = -1.0f;
-        mt[6] = -b;   mt[7] = 1.0f;  mt[8] = -a;
-    } else {
-        mt[0] = -b;   mt[1] = -c;    mt[2] = 1.0f;
-        mt[3] = a;    mt[4] = 1.0f;  mt[5] = c;
-        mt[6] = -1.0f; mt[7] = a;    mt[8] = -b;
-    }
+    carrier_rows<AXIS>(a, b, c, mt);
 }
 
-// 1 / sqrt(mean_9(v^2) + 1e-6) with v_rsq_f32
-__device__ __forceinline__ float rms9_inv_fast(const float v[9]) {
+// mean of the squares of 9 entries plus eps
+__device__ __forceinline__ float ms9(const float v[9]) {
     float s = v[0] * v[0];
 #pragma unroll
     for (int k = 1; k < 9; ++k) s = fmaf(v[k], v[k], s);
-    return __builtin_amdgcn_rsqf(fmaf(s, 1.0f / 9.0f, 1e-6f));
+    return fmaf(s, 1.0f / 9.0f, 1e-6f);
 }
+// 1 / sqrt(x) for x > 0: v_rsq_f32 and one Newton step, which leaves the error
+// of the correctly rounded root and division at a fifth of their operations.
+// x = inf gives 0: the step's 0 * inf is replaced by -1 there, times 0.
+__device__ __forceinline__ float rsq_step(float x) {
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float e = fmaxf(fmaf(-x * y, y, 1.0f), -1.0f);
+    return fmaf(0.5f * y, e, y);
+}
+__device__ __forceinline__ float rms9_inv(const float v[9]) { return rsq_step(ms9(v)); }
+// the same with v_rsq_f32 alone (1 ulp), for the streaming chains
+__device__ __forceinline__ float rms9_inv_fast(const float v[9]) { return __builtin_amdgcn_rsqf(ms9(v)); }
 
 // out = A @ B for row-major 3x3
 __device__ __forceinline__ void mm3(const float A[9], const float B[9], float out[9]) {
@@ -78,14 +95,6 @@ __device__ __forceinline__ void mm3(const float A[9], const float B[9], float ou
 #pragma unroll
         for (int c = 0; c < 3; ++c)
             out[3 * r + c] = fmaf(A[3 * r + 2], B[6 + c], fmaf(A[3 * r + 1], B[3 + c], A[3 * r] * B[c]));
-}
-
-// rms over 9 entries with eps inside the root; returns the rms
-__device__ __forceinline__ float rms9(const float v[9]) {
-    float s = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 9; ++k) s = fmaf(v[k], v[k], s);
-    return sqrtf(s * (1.0f / 9.0f) + 1e-6f);
 }
 
 // M <- M (I - beta/2 (G/s - I)), G = M^T M, s = max(mean(diag G), eps)
@@ -110,9 +119,9 @@ __device__ __forceinline__ void polarm9(float M[9], float beta, float eps) {
     for (int k = 0; k < 9; ++k) M[k] = R[k];
 }
 
-// v <- v / rms9(v)
+// v <- v / rms(v)
 __device__ __forceinline__ void normalize9(float v[9]) {
-    const float inv = 1.0f / rms9(v);
+    const float inv = rms9_inv(v);
 #pragma unroll
     for (int k = 0; k < 9; ++k) v[k] *= inv;
 }

@@ -280,7 +280,7 @@ tria_chunk_scan_kernel(TriaChunkArgs a) {
             // continuation when the previous boundary did not fire)
             float pre[9];
             mm3(Ec, S, pre);
-            const float inv = 1.0f / rms9(pre);
+            const float inv = rms9_inv(pre);
 #pragma unroll
             for (int k = 0; k < 9; ++k) S[k] = pre[k] * inv;
         }
@@ -307,7 +307,7 @@ tria_chunk_scan_kernel(TriaChunkArgs a) {
 #pragma unroll
                 for (int k = 0; k < 9; ++k) u[k] = ld(d + k);
                 mm3(u, S, pre);
-                const float inv = 1.0f / rms9(pre);
+                const float inv = rms9_inv(pre);
 #pragma unroll
                 for (int k = 0; k < 9; ++k) st(d + k, pre[k] * inv);
             }

@@ -741,6 +741,30 @@ def test_temporal_carry(dtype, B, T, H):
     check(e32, ref.temporal_carry_endpoint(D, reset, host(ini), valid), dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,T,H", [(1, 1, 2), (1, 2, 254), (3, 5, 34), (2, 1, 256), (3, 3, 258), (1, 511, 2)])
+@pytest.mark.parametrize("mode", ["init", "seed", "step"])
+def test_tria_depth_element_pairs(dtype, B, T, H, mode):
+    """Two elements per thread (16-bit types, even H, operands aligned to a pair)
+    against one per thread, over whole, ragged and single-pair blocks.  An offset
+    of one element in r takes the call to the form of one element per thread; the
+    arithmetic per element is the same, so the results are the same bits."""
+    from loom_amd import ops
+    g = gen(B * T + H)
+    r, i, o, prev, seed, valid, w = _tria_inputs(g, B, T, H, dtype)
+    off = torch.empty(r.numel() + 1, dtype=dtype, device=DEV)[1:].view(r.shape)
+    off.copy_(r)
+    assert r.data_ptr() % 4 == 0 and off.data_ptr() % 4 == 2
+    rest = {"init": (), "seed": (seed, valid), "step": (prev,)}[mode]
+    fn = {"init": ops.tria_init_gate_forward, "seed": ops.tria_init_seed_gate_forward,
+          "step": ops.tria_step_gate_forward}[mode]
+    for got, want in zip(fn(r, i, o, *rest, w, 0.05, 1), fn(off, i, o, *rest, w, 0.05, 1)):
+        assert torch.equal(got, want)
+    fn = {"init": ops.tria_init_forward, "seed": ops.tria_init_seed_forward, "step": ops.tria_step_forward}[mode]
+    for got, want in zip(fn(r, i, o, *rest, 0.05, 2), fn(off, i, o, *rest, 0.05, 2)):
+        assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("dtype", DTYPES3)
 def test_polarm_and_final_ca(dtype):
     from loom_amd import ops
