@@ -153,12 +153,12 @@ final_ca_tile_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* 
         }
     sum += __shfl_xor(sum, 16, 64);
     sum += __shfl_xor(sum, 32, 64);
-    // a row without a key gives zero
+    // a row without a key gives zero; a NaN weight stays one
     const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
 #pragma unroll
     for (int n = 0; n < NKT; ++n)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) s[n][r] = sum > 0.0f ? s[n][r] * inv : 0.0f;
+        for (int r = 0; r < 4; ++r) s[n][r] *= inv;
     if (lse != nullptr && tid < 16 && live) lse[row] = mx == -INFINITY ? -INFINITY : mx + logf(sum);
 
     for (int sl = wave; sl < slabs; sl += 4) {

@@ -810,6 +810,22 @@ def test_final_ca_sequences(dtype, B, T, K, D):
     check(lse[ok.to(DEV)], wl[ok], torch.float32, rtol=1e-3, atol=1e-3)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_final_ca_tiles_keep_nan(dtype):
+    """A NaN in an allowed key reaches every row that attends to it, and no other."""
+    from loom_amd import ops
+    B, T, K, D = 70, 33, 16, 256
+    g = gen(9)
+    q, k, v = dev(rnd(g, B, T, D), dtype), dev(rnd(g, B, K, D), dtype), dev(rnd(g, B, K, D), dtype)
+    k[3, 5, 7] = float("nan")
+    allowed = torch.ones(B, T, K, dtype=torch.bool)
+    allowed[3, ::2, 5] = False
+    out = host(ops.final_ca_sparse_forward(q, k, v, dev(allowed, torch.bool), D ** -0.5)[0])
+    hit = torch.zeros(B, T, dtype=torch.bool)
+    hit[3, 1::2] = True
+    assert torch.equal(torch.isnan(out).all(-1), hit) and torch.equal(torch.isnan(out).any(-1), hit)
+
+
 def test_final_ca_tiles_strided_with_device_key_count():
     """The 16-row tiles through the cache layout: padded strides, a residual, the
     key count on the device (also zero keys), values past it never read into a row."""
