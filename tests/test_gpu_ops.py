@@ -765,6 +765,25 @@ def test_tria_depth_element_pairs(dtype, B, T, H, mode):
         assert torch.equal(got, want)
 
 
+# one wave, a block of several, more than one round of requests, pairs and single
+# records (odd H, a base off by one element), a row whose scores are far apart
+@pytest.mark.parametrize("dtype", DTYPES3)
+@pytest.mark.parametrize("B,T,H,off", [(1, 1, 1, 0), (2, 1, 2, 0), (3, 2, 65, 0), (2, 2, 1000, 1), (1, 3, 2050, 0),
+                                       (2, 1, 3071, 0), (32, 1, 3072, 0), (1, 1, 9000, 1)])
+def test_slot_pool_sizes(dtype, B, T, H, off):
+    from loom_amd import ops
+    g = gen(B + T + H)
+    buf = dev(rnd(g, B * T * H * 9 + off, scale=2.0), dtype)
+    carry, sw = buf[off:].view(B, T, H, 3, 3), dev(rnd(g, 9, scale=3.0), dtype)
+    pooled, lse = ops.slot_attention_pool_forward(carry, sw)
+    want, want_lse = ref.slot_attention_pool(host(carry), host(sw))
+    check(pooled, want, dtype)
+    check(lse, want_lse, dtype)
+    carry[-1, -1, H // 2, 1, 1] = float("nan")
+    bad = torch.isnan(ops.slot_attention_pool_forward(carry, sw)[0])
+    assert bool(bad[-1, -1].all()) and int(bad.sum()) == 9
+
+
 @pytest.mark.parametrize("dtype", DTYPES3)
 def test_polarm_and_final_ca(dtype):
     from loom_amd import ops
