@@ -1964,10 +1964,8 @@ static int linear_multi_dispatch(const loom_linear_multi_desc& d, hipStream_t st
     return LOOM_OK;
 }
 
-extern "C" int64_t loom_linear_multi_desc_bytes(void) { return (int64_t)sizeof(loom_linear_multi_desc); }
-
-extern "C" int loom_linear_multi(int dtype, const loom_linear_multi_desc* d, void* stream) {
-    clear_error();
+// What loom_linear_multi asks of a descriptor
+static int check_linear_multi(const loom_linear_multi_desc* d) {
     LOOM_CHECK(d != nullptr && d->x != nullptr, "linear_multi: null descriptor or input");
     LOOM_CHECK(d->only_if == nullptr || (d->only_if_n >= 1 && d->only_if_n <= 1024),
                "linear_multi: only_if_n=%lld outside [1, 1024]", (long long)d->only_if_n);
@@ -1986,6 +1984,15 @@ extern "C" int loom_linear_multi(int dtype, const loom_linear_multi_desc* d, voi
                    "linear_multi: the gate applies to single-input segments only");
         LOOM_CHECK(g.gate_p == nullptr || g.gate_ld >= g.n, "linear_multi: gate row stride too small");
     }
+    return LOOM_OK;
+}
+
+extern "C" int64_t loom_linear_multi_desc_bytes(void) { return (int64_t)sizeof(loom_linear_multi_desc); }
+
+extern "C" int loom_linear_multi(int dtype, const loom_linear_multi_desc* d, void* stream) {
+    clear_error();
+    const int rc = check_linear_multi(d);
+    if (rc != LOOM_OK) return rc;
     if (d->m == 0) return LOOM_OK;
     switch (dtype) {
         case LOOM_F32: return linear_multi_dispatch<float>(*d, (hipStream_t)stream);
@@ -2127,6 +2134,8 @@ extern "C" int loom_linear_ln(int dtype, const loom_linear_multi_desc* d, const 
     LOOM_CHECK(out_frag == nullptr || (fused && g.n % 32 == 0 && ((uintptr_t)out_frag & 15) == 0),
                "linear_ln: out_frag needs the bf16 split-K form (m <= 64, aligned) and n %% 32 == 0");
     if (!fused) {
+        LOOM_CHECK(d->x && g.w && d->k >= 1 && d->k2 >= 0 && (d->k2 == 0 || (d->x2 && g.w2)),
+                   "linear_ln: an input or a weight is missing");
         // many rows: the DMA-staged MFMA tiles over both inputs (configuration as
         // big_tile picks it), split-K sums in the workspace, reduced with the bias
         // in the LayerNorm kernel.  Splits: whole rounds of the stages each;
@@ -2160,6 +2169,13 @@ extern "C" int loom_linear_ln(int dtype, const loom_linear_multi_desc* d, const 
                 const int64_t cost = ceil_div(tiles * q, per_cu * (int64_t)device_cus()) * (K / q + 320);
                 if (ns == 0 || cost < best) { ns = q; best = cost; }
             }
+        if (ns == 0) {
+            // no staged form: seg[0].out is part of the call
+            const int rc = check_linear_multi(d);
+            if (rc != LOOM_OK) return rc;
+            LOOM_CHECK(g.ldc == g.n && ldo == g.n, "linear_ln: the unfused path needs dense rows");
+            if (d->m == 0) return LOOM_OK;
+        }
         GemmArgs a{};
         a.X = d->x; a.ldx = d->ldx; a.W = g.w; a.ldw = g.ldw;
         a.X2 = d->k2 > 0 ? d->x2 : nullptr; a.ldx2 = d->ldx2; a.W2 = g.w2; a.ldw2 = g.ldw2;
@@ -2182,12 +2198,10 @@ extern "C" int loom_linear_ln(int dtype, const loom_linear_multi_desc* d, const 
             return launch_splitk_ln(ns, d, workspace, gamma, beta, eps, out, ldo, nullptr, st);
         }
         // y = product (+ bias) into seg.out, then LayerNorm of y
-        int rc = loom_linear_multi(dtype, d, stream);
+        const int rc = loom_linear_multi(dtype, d, stream);
         if (rc != LOOM_OK) return rc;
-        LOOM_CHECK(g.ldc == g.n && ldo == g.n, "linear_ln: the unfused path needs dense rows");
         return loom_add_layernorm(dtype, g.out, nullptr, gamma, beta, out, d->m, g.n, eps, stream);
     }
-    if (d->m == 0) return LOOM_OK;
     LinArgs a{};
     a.X = (const uint16_t*)d->x; a.ldx = d->ldx; a.K = d->k;
     a.X2 = (const uint16_t*)d->x2; a.ldx2 = d->ldx2; a.K2 = d->k2;

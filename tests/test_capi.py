@@ -55,6 +55,38 @@ def test_error_channel_reports_argument_errors():
                   None, p, p, p, None, 1, 1, 3, 0.0375, 0, None)
 
 
+def test_linear_ln_checks_its_descriptor_before_any_launch():
+    """bf16 rows that no staged tile takes (and zero rows) answer as
+    loom_linear_multi does: zero rows are no error, a missing input or weight, a row
+    stride below the row and rows that are not dense are, whichever kernel the
+    product would take (no device here: a launch would be an error of its own)."""
+    from loom_amd import _lib
+
+    def ln(m, ldo=768, null=(), **kw):
+        d = _lib.LinearMultiDesc()
+        d.x, d.ldx, d.k, d.x2, d.ldx2, d.k2, d.m, d.nseg = 256, 768, 768, 256, 768, 768, m, 1
+        s = d.seg[0]
+        s.w, s.ldw, s.w2, s.ldw2, s.out, s.ldc, s.n = 256, 768, 256, 768, 256, 768, 768
+        for k, v in kw.items():
+            setattr(s if hasattr(s, k) else d, k, v)
+        p = ctypes.c_void_p(256)
+        _lib.call("loom_linear_ln", 1, ctypes.byref(d), p, p, 1e-5, p, ldo, p,
+                  _lib.load().loom_linear_ln_workspace_bytes(m, 768), None, None)
+
+    ln(0)
+    ln(0, k2=0, x2=None, w2=None)
+    for m in (0, 100, 4096):
+        for bad in (dict(x2=None), dict(w2=None), dict(x=None), dict(w=None), dict(k=0, k2=0), dict(k2=-64)):
+            with pytest.raises(RuntimeError, match="linear_ln: an input or a weight|linear_multi:"):
+                ln(m, **bad)
+    for bad in (dict(out=None), dict(ldx=760), dict(ldx2=760), dict(ldw=760), dict(ldw2=760)):
+        with pytest.raises(RuntimeError, match="linear_multi:"):
+            ln(100, **bad)
+    for bad in (dict(ldc=776), dict(ldo=776)):
+        with pytest.raises(RuntimeError, match="dense rows"):
+            ln(100, **bad)
+
+
 def test_drop_in_modules_expose_reference_names():
     from kernels.build import EXPORTS, build_or_load
     for ext, names in EXPORTS.items():
