@@ -164,11 +164,13 @@ int64_t loom_linear_multi_desc_bytes(void);
  * descriptor (no gate; N <= 2048): the sublayer tails
  * ln_attn(skip + attn_out) and ln_ffn(skip + ffn_out) of Model.step
  * (loomformer.py:4000, :4045) with both products in one accumulator.  No
- * counterpart in the reference as one call.  bf16 with m <= 64 splits K over
- * blocks, writing fp32 partial sums to the workspace (at least
- * loom_linear_ln_workspace_bytes(m, n), 16-byte aligned), and the LayerNorm
- * kernel adds them up; other cases write x w^T + x2 w2^T + bias to seg[0].out
- * (dense [m, n]) and normalise that.  out_frag (optional, the bf16 split-K form
+ * counterpart in the reference as one call.  bf16 with m <= 64, and with more
+ * rows where a staged tile fits (at least 128 rows, k and k + k2 whole rounds of its stages),
+ * writes fp32 partial sums to the workspace (at least
+ * loom_linear_ln_workspace_bytes(m, n), 16-byte aligned), which the LayerNorm
+ * kernel adds up; seg[0].out is not written then.  Other cases write
+ * x w^T + x2 w2^T + bias to seg[0].out (dense [m, n]) and normalise that (in
+ * bf16 from the sum before it is rounded, where the workspace is given).  out_frag (optional, the bf16 split-K form
  * with n % 32 == 0 only): the result also in fragment-major order. */
 int loom_linear_ln(int dtype, const loom_linear_multi_desc* desc, const float* gamma,
                    const float* beta, float eps, void* out, int64_t ldo, float* workspace,

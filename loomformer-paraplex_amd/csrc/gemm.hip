@@ -2013,12 +2013,13 @@ constexpr int kLnVec = 8;      // 256-column chunks per row: rows of up to 2048
 // step's 32 rows spread over 32 CUs.  Every load of the row (all NS split
 // partials, bias, gamma and beta) is issued before the first add; the row's
 // sum and squared deviation are reduced over the waves through LDS.
-template <typename T, int NS, int KV>
+// Y: the sum itself (with the bias) also goes to y, dense rows of N.
+template <typename T, int NS, int KV, bool Y>
 __global__ void __launch_bounds__(64 * KV)
 splitk_ln_kernel(const float* __restrict__ partial, int64_t ldp,
                  const float* __restrict__ bias, const float* __restrict__ gamma,
                  const float* __restrict__ beta, T* __restrict__ out, int64_t ldo, int64_t rows,
-                 int N, float eps, T* __restrict__ outf) {
+                 int N, float eps, T* __restrict__ outf, T* __restrict__ y) {
     __shared__ float red[2][KV];
     const int64_t row = blockIdx.x;
     const int lane = threadIdx.x & 63, k = threadIdx.x >> 6;
@@ -2039,6 +2040,11 @@ splitk_ln_kernel(const float* __restrict__ partial, int64_t ldp,
 #pragma unroll
     for (int sp = 0; sp < NS; ++sp) {
         x[0] += v[sp].x; x[1] += v[sp].y; x[2] += v[sp].z; x[3] += v[sp].w;
+    }
+    if constexpr (Y) {
+        if (in)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) st(y + row * N + c + e, x[e]);
     }
     float s = in ? (x[0] + x[1]) + (x[2] + x[3]) : 0.0f;
     s = wave_sum(s);
@@ -2065,17 +2071,17 @@ splitk_ln_kernel(const float* __restrict__ partial, int64_t ldp,
     if (!in) return;
     const float g[4] = {gv.x, gv.y, gv.z, gv.w};
     const float e4[4] = {ev.x, ev.y, ev.z, ev.w};
-    T y[4];
+    T o[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        st(&y[e], fmaf((x[e] - mean) * rstd, g[e], e4[e]));
-        out[row * ldo + c + e] = y[e];
+        st(&o[e], fmaf((x[e] - mean) * rstd, g[e], e4[e]));
+        out[row * ldo + c + e] = o[e];
     }
     if (outf != nullptr) {
         // fragment-major copy: piece (row/16, c/32, row%16 + 16*((c%32)/8)), elements c%8 ..
         const int64_t piece = ((row >> 4) * (N >> 5) + (c >> 5)) * 64 + (row & 15) + 16 * ((c & 31) >> 3);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) outf[piece * 8 + (c & 7) + e] = y[e];
+        for (int e = 0; e < 4; ++e) outf[piece * 8 + (c & 7) + e] = o[e];
     }
 }
 
@@ -2083,15 +2089,21 @@ extern "C" int64_t loom_linear_ln_workspace_bytes(int64_t M, int64_t N) {
     return kMaxSplit * M * N * (int64_t)sizeof(float);
 }
 
-// LayerNorm of the ns split-K partial sums (+ bias) of d's product, one block per row
+// LayerNorm of the ns split-K partial sums (+ bias) of d's product, one block per
+// row; y (one partial sum only): the product with its bias, or NULL
 static int launch_splitk_ln(int64_t ns, const loom_linear_multi_desc* d, const float* workspace,
                             const float* gamma, const float* beta, float eps, void* out, int64_t ldo,
-                            void* out_frag, hipStream_t st) {
+                            void* out_frag, void* y, hipStream_t st) {
     const loom_linear_segment& g = d->seg[0];
-#define LOOM_SLN_KV(NS, KV)                                                                   \
-    hipLaunchKernelGGL((splitk_ln_kernel<bf16_t, NS, KV>), dim3((unsigned)d->m), dim3(64 * (KV)), \
+#define LOOM_SLN_Y(NS, KV, Y)                                                                 \
+    hipLaunchKernelGGL((splitk_ln_kernel<bf16_t, NS, KV, Y>), dim3((unsigned)d->m), dim3(64 * (KV)), \
                        0, st, workspace, g.n, g.bias, gamma, beta, (bf16_t*)out, ldo, d->m,     \
-                       (int)g.n, eps, (bf16_t*)out_frag);
+                       (int)g.n, eps, (bf16_t*)out_frag, (bf16_t*)y);
+#define LOOM_SLN_KV(NS, KV)                                                                   \
+    if constexpr (NS == 1) {                                                                  \
+        if (y != nullptr) { LOOM_SLN_Y(NS, KV, true) }                                        \
+        else { LOOM_SLN_Y(NS, KV, false) }                                                    \
+    } else { LOOM_SLN_Y(NS, KV, false) }
 #define LOOM_SLN(NS)                                                                          \
     case NS:                                                                                  \
         if (kv <= 1) { LOOM_SLN_KV(NS, 1) }                                                   \
@@ -2105,6 +2117,7 @@ static int launch_splitk_ln(int64_t ns, const loom_linear_multi_desc* d, const f
         LOOM_SLN(1) LOOM_SLN(2) LOOM_SLN(3) LOOM_SLN(4) LOOM_SLN(5) LOOM_SLN(6) LOOM_SLN(7)
         LOOM_SLN(8)
     }
+#undef LOOM_SLN_Y
 #undef LOOM_SLN_KV
 #undef LOOM_SLN
     return launch_status("loom_linear_ln(layernorm)");
@@ -2182,20 +2195,22 @@ extern "C" int loom_linear_ln(int dtype, const loom_linear_multi_desc* d, const 
         a.K1 = d->k;
         a.M = d->m; a.N = g.n; a.K = K;
         a.partial = workspace; a.ldp = g.n;
-        // direct-fragment tiles: k split inside a block, one partial sum
+        // direct-fragment tiles: k split inside a block, one partial sum (which the
+        // LayerNorm also stores where seg[0].out is part of the call)
         if (aligned && frag_fits<bf16_t, false>(a) && frag_faster(a, false, ns > 0 ? tile : kBigNone, ns > 0 ? ns : 1)) {
             if (a.X2 != nullptr) launch_frag<bf16_t, false, true>(a, st);
             else launch_frag<bf16_t, false, false>(a, st);
             const int rc = launch_status("loom_linear_ln");
             if (rc != LOOM_OK) return rc;
-            return launch_splitk_ln(1, d, workspace, gamma, beta, eps, out, ldo, nullptr, st);
+            return launch_splitk_ln(1, d, workspace, gamma, beta, eps, out, ldo, nullptr,
+                                    ns == 0 ? g.out : nullptr, st);
         }
         if (ns > 0) {
             a.nsplit = (int)ns;
             launch_big<false>(a, tile, ns, st);
             const int rc = launch_status("loom_linear_ln");
             if (rc != LOOM_OK) return rc;
-            return launch_splitk_ln(ns, d, workspace, gamma, beta, eps, out, ldo, nullptr, st);
+            return launch_splitk_ln(ns, d, workspace, gamma, beta, eps, out, ldo, nullptr, nullptr, st);
         }
         // y = product (+ bias) into seg.out, then LayerNorm of y
         const int rc = loom_linear_multi(dtype, d, stream);
@@ -2228,7 +2243,7 @@ extern "C" int loom_linear_ln(int dtype, const loom_linear_multi_desc* d, const 
     launch_skinny_multi(a, grid, (int)ceil_div(d->m, 16), ceil_div(steps, ns), st);
     int rc = launch_status("loom_linear_ln");
     if (rc != LOOM_OK) return rc;
-    return launch_splitk_ln(ns, d, workspace, gamma, beta, eps, out, ldo, out_frag, st);
+    return launch_splitk_ln(ns, d, workspace, gamma, beta, eps, out, ldo, out_frag, nullptr, st);
 }
 
 extern "C" int64_t loom_ffn_decode_desc_bytes(void) { return (int64_t)sizeof(loom_ffn_decode_desc); }

@@ -896,6 +896,29 @@ def test_linear_ln(dtype, M, K2, N):
     check(out, want, dtype)
 
 
+# rows below every staged tile, and a k that is no whole round of a tile's stages
+@pytest.mark.parametrize("M,K,K2,N", [(65, 768, 768, 768), (100, 768, 0, 768), (127, 768, 3072, 200), (500, 832, 256, 520),
+                                      (777, 64, 0, 1028), (300, 768, 832, 96)])
+def test_linear_ln_stores_its_product(M, K, K2, N):
+    """Where no staged tile fits, the product with its bias also goes to seg[0].out,
+    whichever kernel forms it; LayerNorm as ever."""
+    from loom_amd import _lib
+    g = torch.Generator().manual_seed(M + N)
+    r = lambda *s, sc=1.0: (torch.randn(*s, generator=g) * sc).to(DEV, torch.bfloat16)
+    x, w, x2, w2 = r(M, K), r(N, K, sc=K ** -0.5), r(M, max(K2, 1)), r(N, max(K2, 1), sc=max(K2, 1) ** -0.5)
+    b, gam, bet = (torch.randn(N, generator=g).to(DEV) for _ in range(3))
+    y, out = torch.full((M + 1, N), 7.0, device=DEV, dtype=x.dtype), torch.zeros(M, N, device=DEV, dtype=x.dtype)
+    nb = _lib.load().loom_linear_ln_workspace_bytes(M, N)
+    ws = torch.empty(nb // 4, device=DEV)
+    sg = dict(w=w, out=y[:M], bias=b, w2=w2 if K2 else None)
+    d = _lib.linear_multi_desc(x, [sg], x2=x2 if K2 else None)
+    _lib.call("loom_linear_ln", code(x), ctypes.byref(d), P(gam), P(bet), 1e-5, P(out), N, P(ws), nb, None, S(x))
+    pre = host(x) @ host(w).T + host(b) + (host(x2) @ host(w2).T if K2 else 0.0)
+    check(y[:M], pre, x.dtype)
+    assert bool((y[M] == 7.0).all())
+    check(out, torch.nn.functional.layer_norm(pre, (N,), host(gam), host(bet), 1e-5), x.dtype)
+
+
 @pytest.mark.parametrize("M,K2", [(4, 3072), (32, 768), (32, 3072), (20, 0), (64, 768)])
 def test_fragment_major_activations(M, K2):
     """loom_linear_ln's out_frag is the fragment-major copy of its output, and
