@@ -148,18 +148,17 @@ final_ca_tile_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* 
     for (int n = 0; n < NKT; ++n)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            s[n][r] = (mx == -INFINITY || s[n][r] == -INFINITY) ? 0.0f : fexp(s[n][r] - mx);
+            s[n][r] = s[n][r] == -INFINITY ? 0.0f : fexp(s[n][r] - mx);
             sum += s[n][r];
         }
     sum += __shfl_xor(sum, 16, 64);
     sum += __shfl_xor(sum, 32, 64);
-    // a row without a key gives zero; a NaN weight stays one
-    const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
+    const float inv = ca_inv(sum);
 #pragma unroll
     for (int n = 0; n < NKT; ++n)
 #pragma unroll
         for (int r = 0; r < 4; ++r) s[n][r] *= inv;
-    if (lse != nullptr && tid < 16 && live) lse[row] = mx == -INFINITY ? -INFINITY : mx + logf(sum);
+    if (lse != nullptr && tid < 16 && live) lse[row] = ca_lse(mx, sum);
 
     for (int sl = wave; sl < slabs; sl += 4) {
         ca_f32x4 acc[4];

@@ -1086,6 +1086,12 @@ polarm_kernel(const T* __restrict__ in, T* __restrict__ out, const uint8_t* __re
 // time, lanes over D), masked softmax in LDS, then out = sum_j w_j v_j.
 constexpr int kCaMaxK = 1024;
 
+// A row without a key has the sum 0 (every other one holds its maximum's 1): its
+// weights are zero and its lse -inf.  A maximum skips NaN, so it says nothing
+// about them; the sum keeps them, and so do the row's weights and lse.
+__device__ __forceinline__ float ca_inv(float sum) { return sum == 0.0f ? 0.0f : 1.0f / sum; }
+__device__ __forceinline__ float ca_lse(float mx, float sum) { return sum == 0.0f ? -INFINITY : mx + logf(sum); }
+
 // k/v row j of batch b at b*kv_stride_b + j*D; allowed row r at r*allowed_stride.
 // With a residual, out = residual + gamma * attention (TriaFinalCrossAttention
 // adds gamma*out to its input, tria.py:1556-1557, :1593-1595).
@@ -1120,17 +1126,13 @@ final_ca_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __res
         float mx = -INFINITY;
         for (int64_t j = 0; j < K; ++j) mx = fmaxf(mx, wts[j]);
         float sum = 0.0f;
-        if (mx == -INFINITY) {
-            for (int64_t j = 0; j < K; ++j) wts[j] = 0.0f;
-        } else {
-            for (int64_t j = 0; j < K; ++j) {
-                const float e = (wts[j] == -INFINITY) ? 0.0f : expf(wts[j] - mx);
-                wts[j] = e;
-                sum += e;
-            }
-            const float inv = 1.0f / sum;
-            for (int64_t j = 0; j < K; ++j) wts[j] *= inv;
+        for (int64_t j = 0; j < K; ++j) {
+            const float e = (wts[j] == -INFINITY) ? 0.0f : expf(wts[j] - mx);
+            wts[j] = e;
+            sum += e;
         }
+        const float inv = ca_inv(sum);
+        for (int64_t j = 0; j < K; ++j) wts[j] *= inv;
         red[0] = mx;
         red[1] = sum;
     }
@@ -1142,7 +1144,7 @@ final_ca_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __res
         st(out + row * D + d, a);
     }
     if (lse != nullptr && threadIdx.x == 0)
-        lse[row] = red[0] == -INFINITY ? -INFINITY : red[0] + logf(red[1]);
+        lse[row] = ca_lse(red[0], red[1]);
 }
 
 // Vector form for D % 8 == 0, D <= 1536 and 16-byte aligned rows: q is held as
@@ -1206,12 +1208,12 @@ final_ca_vec_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* _
         mx = wave_max(mx);
         float sum = 0.0f;
         for (int64_t j = lane; j < K; j += 64) {
-            const float e = (mx == -INFINITY || wts[j] == -INFINITY) ? 0.0f : fexp(wts[j] - mx);
+            const float e = wts[j] == -INFINITY ? 0.0f : fexp(wts[j] - mx);
             wts[j] = e;
             sum += e;
         }
         sum = wave_sum(sum);
-        const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
+        const float inv = ca_inv(sum);
         for (int64_t j = lane; j < K; j += 64) wts[j] *= inv;
         if (lane == 0) {
             red[0] = mx;
@@ -1247,7 +1249,7 @@ final_ca_vec_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* _
         Vec8<T>::store(out + row * D + ch * 8, a);
     }
     if (lse != nullptr && threadIdx.x == 0)
-        lse[row] = red[0] == -INFINITY ? -INFINITY : red[0] + logf(red[1]);
+        lse[row] = ca_lse(red[0], red[1]);
 }
 
 // Short key lists (16-bit types, K <= kCaRowKeys, D % 8 == 0, D <= 1024): every load of the
@@ -1349,9 +1351,9 @@ final_ca_row_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* _
     if (wid == 0) {
         const float sv = ok ? wts[lane] : -INFINITY;
         const float mx = wave_max(sv);
-        const float e = (mx == -INFINITY || sv == -INFINITY) ? 0.0f : fexp(sv - mx);
+        const float e = sv == -INFINITY ? 0.0f : fexp(sv - mx);
         const float sum = wave_sum(e);
-        if (lane < K) wts[lane] = sum > 0.0f ? e / sum : 0.0f;
+        if (lane < K) wts[lane] = sum == 0.0f ? 0.0f : e / sum;
         if (lane == 0) {
             red[0] = mx;
             red[1] = sum;
@@ -1384,7 +1386,7 @@ final_ca_row_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* _
         Vec8<T>::store(out + row * D + tid * 8, a);
     }
     if (lse != nullptr && tid == 0)
-        lse[row] = red[0] == -INFINITY ? -INFINITY : red[0] + logf(red[1]);
+        lse[row] = ca_lse(red[0], red[1]);
 }
 
 }  // namespace loom

@@ -845,6 +845,30 @@ def test_final_ca_tiles_keep_nan(dtype):
     assert torch.equal(torch.isnan(out).all(-1), hit) and torch.equal(torch.isnan(out).any(-1), hit)
 
 
+# one row and several per block, short and long key lists, widths of each kernel;
+# with one key, every allowed score of a hit row is NaN
+@pytest.mark.parametrize("dtype", DTYPES3)
+@pytest.mark.parametrize("B,T,K,D", [(2, 3, 1, 96), (1, 3, 5, 64), (2, 150, 1, 768), (70, 33, 16, 256), (1, 4, 40, 100),
+                                     (1, 3, 100, 768), (16, 128, 40, 512), (16, 256, 256, 64)])
+def test_final_ca_nan_rows(dtype, B, T, K, D):
+    """A NaN query, and a NaN key where it is allowed, make their rows and those
+    rows' lse NaN; a row without a key gives zeros and -inf all the same."""
+    from loom_amd import ops
+    g = gen(B + T + K + D)
+    q, k, v = dev(rnd(g, B, T, D), dtype), dev(rnd(g, B, K, D), dtype), dev(rnd(g, B, K, D), dtype)
+    q[0, 1], k[B - 1, K - 1] = float("nan"), float("nan")
+    allowed = torch.ones(B, T, K, dtype=torch.bool)
+    allowed[B - 1, ::2, K - 1] = False
+    allowed[0, 2] = False
+    q[0, 2] = float("nan")
+    out, lse = (host(t) for t in ops.final_ca_sparse_forward(q, k, v, dev(allowed, torch.bool), D ** -0.5))
+    none = ~allowed.any(-1)
+    hit = (allowed & (host(q) @ host(k).transpose(1, 2).contiguous()).isnan()).any(-1)
+    assert torch.equal(out.isnan().all(-1), hit) and torch.equal(out.isnan().any(-1), hit)
+    assert torch.equal(lse.isnan(), hit) and torch.equal(lse == -math.inf, none)
+    assert bool((out[none] == 0).all())
+
+
 def test_final_ca_tiles_strided_with_device_key_count():
     """The 16-row tiles through the cache layout: padded strides, a residual, the
     key count on the device (also zero keys), values past it never read into a row."""
