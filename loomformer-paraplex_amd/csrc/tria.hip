@@ -1598,16 +1598,40 @@ static int polarm_dispatch(const void* in, void* out, const uint8_t* mask, int64
     return launch_status("loom_polarm_forward");
 }
 
-// The 16-row tiles of a sequence against one block per row, measured at D =
-// 768: bf16 from more rows than CUs on (256 rows of 16 keys 5.6 us against 5.7,
-// 512 9.5 against 6.0, 16384 of 15 255 against 15.3; the one-row kernel holds a
-// row of up to 64 keys in registers, two blocks per CU); fp32, whose one-row
-// blocks run eight per CU, from rows x keys of 32 K on (14 K 8.5 us against 9.5,
-// 127 K 38 against 16, 245 K 80 against 31).
+// The 16-row tiles of a sequence against one block per row, both timed over rows 130
+// to 16384, 1 to 256 keys, D 64 to 1024.  A tile reads and multiplies 16, 32, 64
+// or 256 keys whatever K is, and 16 rows whatever T is; one round of them takes
+// (D = 768, bf16) 6, 8.5, 13 or 48-57 us.
+//   bf16 (the one-row kernel holds a row of up to 64 keys in registers, two blocks
+//   per CU): up to 32 keys from more rows than CUs on (260 rows of 16 keys 9.2 ->
+//   6.0, 16384 of 15 256 -> 14); 33-64 keys at D > 512 from two rows per CU on (300
+//   rows of 48 keys 11.7 us against 12.6; at D = 1024 11.8 against 15.1; 300 x 2 rows
+//   of 33 keys 22 against 23.6); longer lists where 256 keys are not mostly padding
+//   and the rows fill the chip (600 rows of 100 keys 23.5 against 48, at D = 1024 2400
+//   of 128 78 against 91; 4096 of 256 207 -> 96).
+//   fp32 (one-row blocks run eight per CU): by the work rows x keys that the tile
+//   shares, and only for whole tiles (1024 rows of 48 keys 15.6 against 18.6, 600
+//   of 100 24 against 58; 4096 of 15 22 -> 12, of 100 108 -> 66).
 template <typename T>
-static bool ca_tiles_faster(int64_t rows, int64_t T_, int64_t K) {
-    if (T_ <= 1) return false;
-    return sizeof(T) == 2 ? rows > (int64_t)device_cus() : rows * K >= 32768;
+static bool ca_tiles_faster(int64_t rows, int64_t T_, int64_t K, int64_t D) {
+    const int64_t work = rows * K;
+    if (sizeof(T) == 2) {
+        if (T_ <= 1 || rows <= (int64_t)device_cus()) return false;
+        if (K <= 32) return true;
+        if (K <= 64) return D <= 512 || (rows > 2 * (int64_t)device_cus() && (T_ >= kCaTileRows || K >= 48));
+        return T_ >= kCaTileRows && K >= (D <= 768 ? 112 : 160) && work >= 300000;
+    }
+    if (T_ < kCaTileRows) return false;
+    if (K <= 16) return K >= (D <= 512 ? 2 : D <= 768 ? 4 : 8) && work >= (D <= 768 ? 32768 : 49152);
+    if (K <= 32) return work >= (D <= 256 ? 32768 : 65536);
+    if (K <= 64) return work >= (D <= 256 ? 36000 : 131072);
+    return K >= 80 && work >= 300000;
+}
+
+// whether aligned rows of this shape take the tiles
+template <typename T>
+static bool ca_takes_tiles(int64_t B, int64_t T_, int64_t K, int64_t D) {
+    return D % 64 == 0 && D <= 256 * kCaTileMaxSlabs && K >= 1 && K <= 256 && ca_tiles_faster<T>(B * T_, T_, K, D);
 }
 
 template <typename T>
@@ -1620,7 +1644,7 @@ static int final_ca_dispatch(const void* q, const void* k, const void* v, int64_
                        (uintptr_t)residual) & 15) == 0;
     if constexpr (!std::is_same<T, f16_t>::value) {
         // 16 query rows per block
-        if (vec && D % 64 == 0 && D <= 256 * kCaTileMaxSlabs && K >= 1 && K <= 256 && ca_tiles_faster<T>(B * T_, T_, K)) {
+        if (vec && ca_takes_tiles<T>(B, T_, K, D)) {
             const dim3 grid((unsigned)(B * ceil_div(T_, kCaTileRows)));
             const int ns = D <= 512 ? 2 : D <= 768 ? 3 : 4;
 #define LOOM_CA_TILE(NKT, NS)                                                                    \
@@ -1798,6 +1822,12 @@ extern "C" int loom_final_ca_sparse_forward(int dtype, const void* q, const void
     if (B * T == 0) return LOOM_OK;
     LOOM_DTYPE_SWITCH(dtype, final_ca_dispatch, q, k, v, K * D, allowed, K, nullptr, 0.0f, out, lse,
                       B, T, K, nullptr, D, scale, (hipStream_t)stream)
+}
+
+// For the tests (no part of the C API): whether bf16 or fp32 rows of this shape take
+// the 16-row tiles.
+extern "C" int loom_test_final_ca_tiles(int dtype, int64_t B, int64_t T, int64_t K, int64_t D) {
+    return dtype == LOOM_BF16 ? ca_takes_tiles<bf16_t>(B, T, K, D) : dtype == LOOM_F32 && ca_takes_tiles<float>(B, T, K, D);
 }
 
 extern "C" int loom_final_ca_sparse_strided(int dtype, const void* q, const void* k, const void* v,

@@ -87,6 +87,27 @@ def test_linear_ln_checks_its_descriptor_before_any_launch():
             ln(100, **bad)
 
 
+def test_final_ca_tile_rule():
+    """The shapes whose both kernels were timed take the faster one (256 CUs: no
+    device here), and so does each tile size's test shape."""
+    from loom_amd import _lib
+    takes = _lib.load().loom_test_final_ca_tiles
+    takes.argtypes = [ctypes.c_int] + [ctypes.c_int64] * 4
+    faster = {1: [(8, 2048, 15, 768), (2, 130, 16, 768), (300, 2, 32, 768), (2, 300, 48, 768), (1, 300, 64, 512),
+                  (8, 512, 256, 1024), (8, 512, 120, 768), (130, 17, 15, 768), (32, 130, 33, 320), (30, 140, 17, 1024),
+                  (9, 150, 256, 128), (20, 130, 120, 64)],
+              0: [(8, 512, 15, 768), (8, 2048, 4, 256), (8, 512, 64, 1024), (8, 512, 100, 768), (1, 1024, 48, 256),
+                  (32, 130, 33, 320), (30, 140, 17, 1024), (9, 150, 256, 128), (20, 130, 120, 64)]}
+    slower = {1: [(1, 256, 16, 768), (1, 300, 48, 1024), (2, 130, 48, 768), (300, 2, 100, 768), (2, 300, 100, 512),
+                  (1, 1024, 100, 768), (8, 2048, 100, 1024), (8, 2048, 15, 96), (4096, 1, 15, 768), (8, 2048, 300, 768),
+                  (8, 300, 128, 1024), (300, 2, 33, 1024)],
+              0: [(2, 300, 64, 768), (300, 2, 64, 64), (1, 1024, 32, 1024), (1, 1024, 48, 768), (8, 2048, 2, 1024),
+                  (2, 300, 100, 1024), (1, 256, 256, 1024), (1, 1024, 33, 256)]}
+    for code in (0, 1):
+        assert [s for s in faster[code] if not takes(code, *s)] == []
+        assert [s for s in slower[code] if takes(code, *s)] == []
+
+
 def test_drop_in_modules_expose_reference_names():
     from kernels.build import EXPORTS, build_or_load
     for ext, names in EXPORTS.items():

@@ -809,11 +809,13 @@ def test_polarm_and_final_ca(dtype):
 
 
 # the 16-row tiles of the sequence form: 1 to 16 key tiles (and one key more than
-# a tile), ragged rows, 1 to 4 slabs per wave, and the widths and key counts that
-# stay with the one-row kernels (D = 1536, 96 and 1100)
+# a tile) in both types, ragged rows, 1 to 4 slabs per wave, and the widths, key counts
+# and rows that stay with the one-row kernels (D = 1536, 96 and 1100, few rows
+# of many keys)
 @pytest.mark.parametrize("dtype", DTYPES3)
 @pytest.mark.parametrize("B,T,K,D", [(150, 2, 1, 64), (130, 17, 15, 768), (70, 33, 16, 512), (16, 130, 17, 1024),
                                      (26, 40, 33, 320), (12, 31, 100, 768), (9, 16, 256, 128), (1, 300, 120, 256),
+                                     (32, 130, 33, 320), (30, 140, 17, 1024), (9, 150, 256, 128), (20, 130, 120, 64),
                                      (60, 5, 9, 1536), (20, 20, 9, 96), (20, 20, 9, 1100)])
 def test_final_ca_sequences(dtype, B, T, K, D):
     from loom_amd import ops
