@@ -1673,44 +1673,104 @@ static void launch_frag_cfg(const GemmArgs& a, hipStream_t st) {
     const dim3 grid((unsigned)(ceil_div(a.M, C::TM) * ceil_div(a.N, C::TN)));
     hipLaunchKernelGGL((gemm_frag_kernel<T, MT, NT, KW, U, GATHER, DUAL>), grid, dim3(C::THREADS), 0, st, a);
 }
+// k parts of the 64 x 64 tiles: eight (one block per CU) or four (two blocks per
+// CU), whichever fills its rounds better
+static int frag_wide_parts(int64_t M, int64_t N) {
+    const int64_t n = ceil_div(M, 64) * ceil_div(N, 64), c = device_cus();
+    return n <= c || ceil_div(n, c) < 2 * ceil_div(n, 2 * c) ? 8 : 4;
+}
 template <typename T, bool GATHER, bool DUAL>
 static void launch_frag(const GemmArgs& a, hipStream_t st) {
     const FragTile t = frag_tile<T>(a.M, a.N, a.K, GATHER, a.Hq);
-    if (t.tm == 64 && t.tn == 64) {
-        // eight k parts (one block per CU) or four (two blocks per CU), whichever
-        // fills its rounds better
-        const int64_t n = ceil_div(a.M, 64) * ceil_div(a.N, 64), c = device_cus();
-        if (n <= c || ceil_div(n, c) < 2 * ceil_div(n, 2 * c)) return launch_frag_cfg<T, 4, 4, 8, 1, GATHER, DUAL>(a, st);
-        return launch_frag_cfg<T, 4, 4, 4, 1, GATHER, DUAL>(a, st);
-    }
+    if (t.tm == 64 && t.tn == 64)
+        return frag_wide_parts(a.M, a.N) == 8 ? launch_frag_cfg<T, 4, 4, 8, 1, GATHER, DUAL>(a, st)
+                                              : launch_frag_cfg<T, 4, 4, 4, 1, GATHER, DUAL>(a, st);
     if (t.tm == 64) return launch_frag_cfg<T, 4, 2, sizeof(T) == 4 ? 4 : 8, 1, GATHER, DUAL>(a, st);
     if (t.tn == 32) return launch_frag_cfg<T, 2, 2, 4, 2, GATHER, DUAL>(a, st);
     if (t.tm == 32) return launch_frag_cfg<T, 2, 1, 8, 2, GATHER, DUAL>(a, st);
     launch_frag_cfg<T, 1, 1, 16, 1, GATHER, DUAL>(a, st);
 }
 
-// bf16: the direct-fragment kernels or the DMA-staged tiles, by the estimate
-// above and, for the staged tiles, per round of the CUs 6000 ns + 640 per 64 of
-// K (1120 for the gather).  Measured: 999 x 768 x 3072 20.9 against 37 us, 512 x
-// 3072 x 768 12.0 against 13.4, 2048 x 3072 x 768 35 against 16.6.
-static bool frag_faster(const GemmArgs& a, bool gather, BigTile tile, int64_t nsplit) {
+// The DMA-staged tiles' time in ns, one k split: per round of the CUs a fixed part
+// and one per k (the gather's packed columns come in more and shorter runs).
+// Measured (estimated) us of one round: 128 x 128 K = 512 8.2 (8.1), 1024 11.7
+// (12.0), 2048 18.5 (19.8), 4096 34 (35); 256 x 128 K = 768 12.4 (12.2), 3072 36.3
+// (35.7); 128 x 192 K = 768 12.2 (12.0), 3072 33-39 (34.1); gather 128 x 128 K =
+// 768 14.6 (14.4), 256 x 128 768 18.2 (17.8), 1152 24.7 (24.7), 1536 32 (31.6), 128 x
+// 192 1152 23.5 (23.0).
+static int64_t staged_ns(BigTile tile, int64_t M, int64_t N, int64_t K, bool gather) {
+    const int64_t bm = tile == kBigSmall || tile == kBigTallS || tile == kBigWide ? 128 : 256;
+    const int64_t per_cu = tile == kBigSmall || tile == kBigTallS ? 2 : 1;
+    int64_t fixed = gather ? 4000 : 4400, per10 = gather ? 180 : 102;   // per10: ns per ten k
+    if (tile == kBigSmall) { fixed = gather ? 4000 : 4200; per10 = gather ? 135 : 76; }
+    if (tile == kBigTall) per10 = gather ? 200 : 120;
+    if (tile == kBigTallS) { fixed = gather ? 4000 : 4600; per10 = gather ? 165 : 96; }
+    const int64_t blocks = ceil_div(M, bm) * ceil_div(N, big_tile_n(tile));
+    return ceil_div(blocks, per_cu * (int64_t)device_cus()) * (fixed + K * per10 / 10);
+}
+
+// A direct-fragment product's time for this comparison: frag_tile's, and more for
+// further rounds, two of which run as one of two blocks per CU (measured, estimated
+// us: two rounds 1024 x 1152 x 768 12.6, 11.9; three 999 x 3072 x 1152 of the gather
+// 26.5, 24.4, 1280 x 2048 x 768 of it 19.7, 18.3)
+static int64_t frag_ns(const GemmArgs& a, bool gather) {
+    const FragTile t = frag_tile<bf16_t>(a.M, a.N, a.K, gather, a.Hq);
+    const int64_t rounds = ceil_div(ceil_div(a.M, t.tm) * ceil_div(a.N, t.tn), (int64_t)device_cus());
+    return t.ns + (rounds <= 2 ? 700 : 1500) * (rounds - 1);
+}
+
+// bf16: the direct-fragment kernels or the DMA-staged tiles.  Over 14 widths of 512
+// to 4096 x K 512 to 4096, 65 to 4096 rows, both modes, and the gather at three head
+// sizes, no product takes the direct-fragment kernels where they are more than 2%
+// slower (with one estimate for every tile, 52 of 1000 did: 1024 x 2048 x 512 9.9 us
+// against 8.3, 3072 x 512 x 2048 28.5 against 19).
+static bool frag_faster(const GemmArgs& a, bool gather, BigTile tile) {
+    return tile == kBigNone || frag_ns(a, gather) < staged_ns(tile, a.M, a.N, a.K, gather);
+}
+
+// The same for the two-input product with LayerNorm, whose staged tiles also write
+// nsplit partial sums for the LayerNorm to read: 6000 ns + 640 per 64 of k a round
+static bool frag_faster_ln(const GemmArgs& a, BigTile tile, int64_t nsplit) {
     if (tile == kBigNone) return true;
     const int64_t bm = tile == kBigSmall || tile == kBigTallS || tile == kBigWide ? 128 : 256;
     const int64_t per_cu = tile == kBigSmall || tile == kBigTallS ? 2 : 1;
     const int64_t blocks = ceil_div(a.M, bm) * ceil_div(a.N, big_tile_n(tile)) * nsplit;
     const int64_t rounds = ceil_div(blocks, per_cu * (int64_t)device_cus());
-    return frag_tile<bf16_t>(a.M, a.N, a.K, gather, a.Hq).ns < rounds * (6000 + a.K / nsplit * (gather ? 1120 : 640) / 64);
+    return frag_tile<bf16_t>(a.M, a.N, a.K, false, 0).ns < rounds * (6000 + a.K / nsplit * 640 / 64);
 }
 
-// whether run_gemm gives a bf16 product of more than 64 rows to the
-// direct-fragment kernels
-static bool linear_takes_frag(const GemmArgs& a) {
-    return a.M > 64 && frag_fits<bf16_t, false>(a) &&
-           frag_faster(a, false, big_tile(a.M, a.N, a.K, false, 0), 1);
+// whether run_gemm gives a bf16 product to the direct-fragment kernels.  Up to 24
+// rows of few k stay with the skinny kernel (2048 x 512 and 17 rows 3.6 us
+// against 3.8; 24 x 512 x 512 equal), up to 20 of many columns too (3072 x 768 and
+// 17 rows 3.9 against 4.0); other products of 17 to 64 rows gain (3072 x 768: M = 32
+// 4.8 -> 4.5 us, 64 6.7 -> 4.9; 768 x 3072: 10.7 -> 6.6, 16.6 -> 7.0).  staged: only
+// where no staged tile fits.
+static bool takes_frag(const GemmArgs& a, bool gather, BigTile tile, bool staged) {
+    if (a.M <= (a.K <= 512 ? 24 : a.K <= 768 && a.N >= 2048 ? 20 : 16)) return false;
+    return a.M <= 64 || (staged ? tile == kBigNone : frag_faster(a, gather, tile));
+}
+
+// whether loom_linear_multi's products of more than 64 rows may take the
+// direct-fragment kernels.  One launch for two products takes the staged tiles, and
+// gives the bits of the products alone, so the line is one that each product
+// sees by itself: W_real and the history slot (3072 + 1536 columns of 768) in one
+// launch of staged tiles against two of direct fragments M = 128 11.1 and 10.5 us,
+// 300 15.9 and 13.5, 384 15.2 and 19.2, 768 17.4 and 32.1; 6144 of 1024 M = 256 13.3
+// and 13.8.
+static bool multi_takes_frag(int64_t m, int64_t k) { return m <= 320 && m * k <= 320 * 768; }
+static bool multi_product_takes_frag(const GemmArgs& a) {
+    return frag_fits<bf16_t, false>(a) && takes_frag(a, false, big_tile(a.M, a.N, a.K, false, 0), !multi_takes_frag(a.M, a.K));
+}
+
+// estimated ns of a bf16 product by itself
+static int64_t product_ns(const GemmArgs& a) {
+    const BigTile tile = big_tile(a.M, a.N, a.K, false, 0);
+    const int64_t f = frag_fits<bf16_t, false>(a) ? frag_ns(a, false) : INT64_MAX / 4;
+    return tile == kBigNone ? f : std::min(f, staged_ns(tile, a.M, a.N, a.K, false));
 }
 
 template <typename T, bool GATHER>
-static int run_gemm(const GemmArgs& a, hipStream_t st, const char* what) {
+static int run_gemm(const GemmArgs& a, hipStream_t st, const char* what, bool staged = false) {
     if (a.M == 0 || a.N == 0) return LOOM_OK;
     if constexpr (sizeof(T) == 2 && std::is_same<T, bf16_t>::value) {
         bool sk = a.M <= 64 && a.K % 8 == 0 && a.ldw % 8 == 0 && ((uintptr_t)a.W & 15) == 0;
@@ -1720,11 +1780,8 @@ static int run_gemm(const GemmArgs& a, hipStream_t st, const char* what) {
                   (uintptr_t)a.src[3] | (uintptr_t)a.src[4]) % 16 == 0;
         else
             sk = sk && a.ldx % 8 == 0 && ((uintptr_t)a.X & 15) == 0;
-        // more than 16 rows: the direct-fragment tiles, which split the rows too
-        // (3072 x 768: M = 32 4.8 -> 4.5 us, 64 6.7 -> 4.9; 768 x 3072: 10.7 ->
-        // 6.6, 16.6 -> 7.0; one 16-row tile: 7.9 us here)
-        if (a.M > 16 && frag_fits<T, GATHER>(a) &&
-            (a.M <= 64 || frag_faster(a, GATHER, big_tile(a.M, a.N, a.K, GATHER, a.Hq), 1))) {
+        // the direct-fragment tiles, which split the rows too
+        if (frag_fits<T, GATHER>(a) && takes_frag(a, GATHER, big_tile(a.M, a.N, a.K, GATHER, a.Hq), staged)) {
             launch_frag<T, GATHER, false>(a, st);
             return launch_status(what);
         }
@@ -1822,6 +1879,33 @@ static int beta_dispatch(const GemmArgs& a, void* r_pack, int64_t QH, hipStream_
 }  // namespace loom
 
 using namespace loom;
+
+// For the tests (no part of the C API): the kernel that an aligned product of more
+// than 8 rows takes.  Direct fragments 100 * tile rows + tile columns, + 10000 * k
+// parts for 64 x 64; staged tiles 1 256 x 128, 2 128 x 128, 3 128 x 256, 4 256 x 192,
+// 5 128 x 192; 0 another.  head_dim > 0: the gather of loom_beta_forward (N =
+// hidden, eight q heads); multi: as one of loom_linear_multi's products.
+extern "C" int loom_test_gemm_kernel(int dtype, int64_t M, int64_t N, int64_t K, int64_t head_dim, int multi) {
+    GemmArgs a{};
+    void* const at = (void*)256;
+    a.X = a.W = at;
+    for (auto& s : a.src) s = at;
+    a.M = M; a.N = N; a.K = a.ldx = a.ldw = K;
+    a.HD = head_dim; a.Nm = 8 * head_dim; a.Hq = N / 8;
+    const bool g = head_dim > 0;
+    const auto frag = [&](FragTile t) {
+        const int parts = t.tm == 64 && t.tn == 64 ? frag_wide_parts(M, N) : 0;
+        return 10000 * parts + 100 * t.tm + t.tn;
+    };
+    if (dtype == LOOM_F32) {
+        const bool fits = g ? frag_fits<float, true>(a) : frag_fits<float, false>(a);
+        return fits && M > 8 ? frag(frag_tile<float>(M, N, K, g, a.Hq)) : 0;
+    }
+    const BigTile tile = big_tile(M, N, K, g, a.Hq);
+    const bool fits = g ? frag_fits<bf16_t, true>(a) : frag_fits<bf16_t, false>(a);
+    if (fits && takes_frag(a, g, tile, multi != 0 && !multi_takes_frag(M, K))) return frag(frag_tile<bf16_t>(M, N, K, g, a.Hq));
+    return M > 64 ? (int)tile : 0;
+}
 
 extern "C" int loom_linear(int dtype, const void* A, int64_t lda, const void* W, int64_t ldw,
                            const float* bias, const void* gate_p, float gate_alpha,
@@ -1929,7 +2013,8 @@ static int linear_multi_dispatch(const loom_linear_multi_desc& d, hipStream_t st
         b.W = g1.w; b.ldw = g1.ldw; b.N = g1.n;
         // (where a product alone takes the direct-fragment tiles, both run alone:
         // one launch gives the bits of the separate products)
-        if (tile != kBigNone && g0.n % big_tile_n(tile) == 0 && !linear_takes_frag(a) && !linear_takes_frag(b)) {
+        if (tile != kBigNone && g0.n % big_tile_n(tile) == 0 && !multi_product_takes_frag(a) &&
+            !multi_product_takes_frag(b)) {
             a.out = g0.out; a.ldc = g0.ldc;
             a.bias = g0.bias; a.gate_p = g0.gate_p; a.gate_alpha = g0.gate_alpha;
             a.M = d.m; a.N = g0.n + g1.n; a.K = d.k;
@@ -1949,7 +2034,7 @@ static int linear_multi_dispatch(const loom_linear_multi_desc& d, hipStream_t st
                        "linear_multi: over 64 rows a gate needs the output's row stride (gate_ld %lld, ldc %lld)",
                        (long long)g.gate_ld, (long long)g.ldc);
             a.bias = g.bias; a.gate_p = g.gate_p; a.gate_alpha = g.gate_alpha;
-            int rc = run_gemm<T, false>(a, st, "loom_linear_multi");
+            int rc = run_gemm<T, false>(a, st, "loom_linear_multi", !multi_takes_frag(d.m, d.k));
             if (rc != LOOM_OK) return rc;
             continue;
         }
@@ -2197,7 +2282,7 @@ extern "C" int loom_linear_ln(int dtype, const loom_linear_multi_desc* d, const 
         a.partial = workspace; a.ldp = g.n;
         // direct-fragment tiles: k split inside a block, one partial sum (which the
         // LayerNorm also stores where seg[0].out is part of the call)
-        if (aligned && frag_fits<bf16_t, false>(a) && frag_faster(a, false, ns > 0 ? tile : kBigNone, ns > 0 ? ns : 1)) {
+        if (aligned && frag_fits<bf16_t, false>(a) && frag_faster_ln(a, ns > 0 ? tile : kBigNone, ns > 0 ? ns : 1)) {
             if (a.X2 != nullptr) launch_frag<bf16_t, false, true>(a, st);
             else launch_frag<bf16_t, false, false>(a, st);
             const int rc = launch_status("loom_linear_ln");
@@ -2429,6 +2514,21 @@ extern "C" int loom_gemm_shared_tiles(int on) {
     return g_shared_tiles.exchange(on != 0 ? 1 : 0);
 }
 
+// One launch, or the products by themselves and the RoPE launch: the staged tiles'
+// estimate with the RoPE epilogue's registers to move (256 x 192 tiles 15000 ns more,
+// 128 x 192 6500), against the products' and 3000 ns + 1 ns per 900 elements
+// of q, k and v (read and written; rows of 1152 + 1536 columns of 768, 128 x 192 tiles: 512 rows
+// 19.2 us against 17.7, 768 20.3 and 22.1, 1024 21.4 and 26.5; without the history
+// columns 512 18.7 and 10.5, 1536 19.8 and 16.4, 2048 19.4 and 24.9)
+static bool prefill_qkv_fused_faster(const GemmArgs& qkv, const void* w_hist, int64_t n_hist, bool shared) {
+    GemmArgs h = qkv;
+    h.W = w_hist;
+    h.N = n_hist;
+    const int64_t cols = qkv.N + (w_hist != nullptr ? n_hist : 0);
+    const int64_t one = staged_ns(shared ? kBigTallS : kBigTall, qkv.M, cols, qkv.K, false) + (shared ? 6500 : 15000);
+    return one <= product_ns(qkv) + (w_hist != nullptr ? product_ns(h) : 0) + 3000 + qkv.M * qkv.N / 900;
+}
+
 extern "C" int loom_prefill_qkv(int dtype, const void* x, int64_t ldx, const void* w_qkv,
                                 const void* w_hist, void* hist_out, int64_t hist_ld, int64_t n_hist,
                                 void* qkv_scratch, void* q_out, void* k_cache, void* v_cache,
@@ -2459,13 +2559,12 @@ extern "C" int loom_prefill_qkv(int dtype, const void* x, int64_t ldx, const voi
     const bool shared = g_shared_tiles.load(std::memory_order_relaxed) != 0;
     GemmArgs qkv{};
     qkv.X = x; qkv.ldx = ldx; qkv.W = w_qkv; qkv.ldw = K; qkv.M = M; qkv.N = QKV; qkv.K = K;
-    // (few rows: the direct-fragment product and the separate RoPE launch)
-    const bool fused = !linear_takes_frag(qkv) && dtype == LOOM_BF16 && HD == 96 && QKV % BgTall::BG_N == 0 &&
+    const bool fused = dtype == LOOM_BF16 && HD == 96 && QKV % BgTall::BG_N == 0 &&
                        (shared ? big_fits<BgTallS>(M, K, false, 0) : big_fits<BgTall>(M, K, false, 0)) &&
                        K % 8 == 0 && ldx % 8 == 0 &&
                        (a16 & 15) == 0 && (a8 & 7) == 0 && cache_stride_b % 4 == 0 &&
                        cache_stride_t % 4 == 0 && cache_stride_h % 4 == 0 &&
-                       (w_hist == nullptr || hist_ld % 4 == 0);
+                       (w_hist == nullptr || hist_ld % 4 == 0) && prefill_qkv_fused_faster(qkv, w_hist, n_hist, shared);
     if (fused) {
         GemmArgs a{};
         a.X = x; a.ldx = ldx; a.W = w_qkv; a.ldw = K; a.out = qkv_scratch; a.ldc = QKV;

@@ -87,6 +87,41 @@ def test_linear_ln_checks_its_descriptor_before_any_launch():
             ln(100, **bad)
 
 
+def test_product_kernel_rule():
+    """Products whose kernels were timed against each other take the faster one
+    (256 CUs: no device here); loom_linear_multi's products of many rows take the
+    staged tiles, alone as in one launch."""
+    from loom_amd import _lib
+    lib = _lib.load()
+    kernel = lib.loom_test_gemm_kernel
+    kernel.argtypes = [ctypes.c_int] + [ctypes.c_int64] * 4 + [ctypes.c_int]
+    def of(*s, hd=0, multi=0, dtype=1, shared=0):
+        prev = lib.loom_gemm_shared_tiles(shared)
+        try:
+            return kernel(dtype, *s, hd, multi)
+        finally:
+            lib.loom_gemm_shared_tiles(prev)
+    # staged tiles faster than direct fragments
+    for s in [(1024, 2048, 512), (640, 2048, 512), (512, 4096, 1024), (3072, 512, 2048), (4096, 512, 2048),
+              (2048, 1024, 4096), (2048, 1024, 1024), (4096, 512, 512)]:
+        assert of(*s) == 2, s
+    assert of(8192, 3072, 768) == 3 and of(2048, 768, 3072) == 1
+    for M in (768, 777, 1024):
+        assert of(M, 3072, 1152, hd=96, shared=1) == 5
+    # and slower
+    for s in [(999, 768, 3072), (512, 768, 768), (1024, 768, 768), (512, 3072, 768), (1024, 512, 2048), (512, 1024, 1024)]:
+        assert of(*s) > 100, s
+    assert of(600, 4096, 1536, hd=128) > 100 and of(333, 3072, 1152, hd=96, shared=1) > 100
+    # few rows: the skinny kernel up to 24 rows of few k
+    assert of(17, 2048, 512) == 0 and of(24, 512, 512) == 0 and of(20, 3072, 768) == 0
+    assert of(25, 2048, 512) > 100 and of(17, 768, 768) > 100 and of(17, 768, 3072) > 100
+    # two products in one launch, and each by itself
+    for M in (384, 512, 768, 1024):
+        for N in (3072, 1536, 4608):
+            assert of(M, N, 768, multi=1) in (1, 2, 3, 4)
+    assert of(300, 4608, 768, multi=1) > 100 and of(256, 6144, 1024, multi=1) < 100
+
+
 def test_final_ca_tile_rule():
     """The shapes whose both kernels were timed take the faster one (256 CUs: no
     device here), and so does each tile size's test shape."""
