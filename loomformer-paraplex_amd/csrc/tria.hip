@@ -461,19 +461,21 @@ struct RawRecs {
 
 // One block per row: softmax over H of <score_w, vec C_h>; each thread keeps
 // an online (max, sum, 9-slot) state over its h's, then the block merges.  A row
-// is one chain of memory round trips and a window has only a block per
-// sequence, so the block is as wide as H allows (up to kPoolThreads) and a
-// thread requests U pieces of CH records before it uses one.  The merges rescale
-// once to the common maximum and then only add; an exponential pair in each
-// shuffle round and a last thread that summed the waves alone took 9.8 us against
-// 8.2 (kernel trace, 32 rows of 3072 in bf16).  A whole fire window of 32 x 128 is
-// 169.9 us against 172.4 with 256 threads and a record at a time.
-constexpr int kPoolThreads = 1024;
+// is one chain of memory round trips: a thread requests kPoolUnits pieces of CH
+// records before it uses one (past the row the last piece again, so a block is no
+// wider than pieces to request), and blocks of up to 256 threads leave a CU room
+// for several; 512 where rows are long and the CUs have one each.  bf16, us with a
+// record at a time in 256 threads, with blocks as wide as the row (up to 1024), and
+// so: 32 rows of 3072 7.3, 6.5, 5.5; 480 of 2048 7.3, 10.9, 5.9; 2048 of 3072 23.3,
+// 39.6, 20.0; 32 of 8192 12.3, 7.2, 7.1.  The merges rescale once to the common
+// maximum and then only add.
+constexpr int kPoolThreads = 512;
+template <int CH> constexpr int kPoolUnits = CH == 2 ? 2 : 3;
 template <typename T, int CH>
 __global__ void __launch_bounds__(kPoolThreads)
 slot_pool_kernel(const T* __restrict__ carry, const T* __restrict__ score_w,
                  T* __restrict__ pooled, T* __restrict__ lse, int64_t H) {
-    constexpr int U = CH == 2 ? 2 : 3;
+    constexpr int U = kPoolUnits<CH>;
     __shared__ float red[kPoolThreads / 64][11];
     const int64_t row = blockIdx.x;
     const T* base = carry + row * H * 9;
@@ -1548,7 +1550,8 @@ static int slot_pool_dispatch(const void* carry, const void* sw, void* pooled, v
                               int64_t rows, int64_t H, hipStream_t st) {
     auto launch = [&](auto records) {
         constexpr int CH = decltype(records)::value;
-        const int64_t threads = std::min((int64_t)kPoolThreads, 64 * ceil_div(H / CH, (int64_t)64));
+        const int64_t units = H / CH, cap = units >= 2048 && rows <= (int64_t)device_cus() ? kPoolThreads : 256;
+        const int64_t threads = std::min(cap, 64 * ceil_div(units, (int64_t)(64 * kPoolUnits<CH>)));
         hipLaunchKernelGGL((slot_pool_kernel<T, CH>), dim3((unsigned)rows), dim3((unsigned)threads), 0, st,
                            (const T*)carry, (const T*)sw, (T*)pooled, (T*)lse, H);
     };

@@ -765,11 +765,13 @@ def test_tria_depth_element_pairs(dtype, B, T, H, mode):
         assert torch.equal(got, want)
 
 
-# one wave, a block of several, more than one round of requests, pairs and single
+# one wave, a block of several (up to 256 threads, and 512), more than one round of
+# requests, more rows than CUs, pairs and single
 # records (odd H, a base off by one element), a row whose scores are far apart
 @pytest.mark.parametrize("dtype", DTYPES3)
 @pytest.mark.parametrize("B,T,H,off", [(1, 1, 1, 0), (2, 1, 2, 0), (3, 2, 65, 0), (2, 2, 1000, 1), (1, 3, 2050, 0),
-                                       (2, 1, 3071, 0), (32, 1, 3072, 0), (1, 1, 9000, 1)])
+                                       (2, 1, 3071, 0), (32, 1, 3072, 0), (1, 1, 9000, 1),
+                                       (300, 1, 129, 0), (5, 60, 500, 0), (290, 1, 4100, 0), (2, 1, 386, 0)])
 def test_slot_pool_sizes(dtype, B, T, H, off):
     from loom_amd import ops
     g = gen(B + T + H)
