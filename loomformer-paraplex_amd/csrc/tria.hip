@@ -657,7 +657,10 @@ temporal_carry_kernel(const T* __restrict__ depth, const uint8_t* __restrict__ r
 // 3072 in bf16 against 67 with a dependent reset byte per step and libm's
 // normalisation (4.9 TB/s, the rate of a large copy); four chains per lane
 // take 57 (176 registers, two waves per SIMD).
-template <typename T, int CH>
+// STEPS > 0: quarters of at most STEPS steps, all of them in flight and nothing
+// requested again (of one to six tokens the ring requested eight steps for one or
+// two: 32 x 3072 in fp32 9.1 -> 12.2 us for one token, 11.5 -> 12.2 for five).
+template <typename T, int CH, int STEPS>
 __global__ void __launch_bounds__(kTriaThreads)
 temporal_endpoint_quarters_kernel(const T* __restrict__ depth, const uint8_t* __restrict__ reset,
                                   const T* __restrict__ initial, const uint8_t* __restrict__ init_valid,
@@ -688,23 +691,26 @@ temporal_endpoint_quarters_kernel(const T* __restrict__ depth, const uint8_t* __
     const int64_t step = H * 9;
     const T* p = depth + (b * T_ * H + h) * 9;
     const uint8_t* rp = reset + b * T_;
-    RawRecs<T, CH> buf[kPrefetch];
-    uint8_t rbuf[kPrefetch];
+    constexpr int PF = STEPS > 0 ? STEPS : kPrefetch;
+    RawRecs<T, CH> buf[PF];
+    uint8_t rbuf[PF];
     const int64_t t_safe = max(t_end - 1, (int64_t)0);
     auto fetch = [&](int u, int64_t t) {
         const int64_t tc = min(t, t_safe);
         buf[u].load(p + tc * step);
         rbuf[u] = rp[tc];
     };
+    if (STEPS != 1 || T_ > 1)                       // (one token is the last step alone)
 #pragma unroll
-    for (int u = 0; u < kPrefetch; ++u) fetch(u, t_begin + u);
-    for (int64_t t0 = t_begin; t0 < t_begin + L; t0 += kPrefetch) {
+        for (int u = 0; u < PF; ++u) fetch(u, t_begin + u);
+    for (int64_t t0 = t_begin; t0 < t_begin + L; t0 += PF) {
+        if (STEPS == 1 && T_ == 1) break;
 #pragma unroll
-        for (int u = 0; u < kPrefetch; ++u) {
+        for (int u = 0; u < PF; ++u) {
             float loc[CH][9];
             buf[u].to_float(loc);
             const bool rs = rbuf[u] != 0;
-            fetch(u, t0 + u + kPrefetch);
+            if constexpr (STEPS == 0) fetch(u, t0 + u + PF);
             if (t0 + u < t_end) {
                 cut = cut || rs;
 #pragma unroll
@@ -1578,10 +1584,17 @@ static int temporal_dispatch(bool full, const void* depth, const uint8_t* reset,
         // chains per lane when H is even and the tensors 4-byte aligned
         auto launch = [&](auto chains) {
             constexpr int CH = decltype(chains)::value;
-            hipLaunchKernelGGL((temporal_endpoint_quarters_kernel<T, CH>),
-                               dim3((unsigned)ceil_div(B * H / CH, kTriaThreads / 4)), blk, 0, st,
-                               (const T*)depth, reset, (const T*)initial, valid, (T*)endpoint, end32, B,
-                               T_, H);
+            auto go = [&](auto steps) {
+                hipLaunchKernelGGL((temporal_endpoint_quarters_kernel<T, CH, decltype(steps)::value>),
+                                   dim3((unsigned)ceil_div(B * H / CH, kTriaThreads / 4)), blk, 0, st,
+                                   (const T*)depth, reset, (const T*)initial, valid, (T*)endpoint, end32, B,
+                                   T_, H);
+            };
+            const int64_t L = (T_ + 3) / 4;         // steps of a quarter
+            if (L <= 1) go(std::integral_constant<int, 1>{});
+            else if (L <= 2) go(std::integral_constant<int, 2>{});
+            else if (L <= 4) go(std::integral_constant<int, 4>{});
+            else go(std::integral_constant<int, 0>{});
         };
         const uintptr_t at = (uintptr_t)depth | (uintptr_t)initial;
         if (sizeof(T) == 2 && H % 2 == 0 && at % 4 == 0)

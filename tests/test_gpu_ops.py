@@ -716,7 +716,10 @@ def test_gate_mix_and_slot_pool(dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES3)
-@pytest.mark.parametrize("B,T,H", [(3, 9, 6), (2, 64, 1000), (1, 1, 5), (1, 3, 7), (4, 128, 3072)])
+# the endpoint's quarters of one, up to two, up to four and more steps, pairs and
+# single chains
+@pytest.mark.parametrize("B,T,H", [(3, 9, 6), (2, 64, 1000), (1, 1, 5), (1, 3, 7), (4, 128, 3072), (3, 1, 130), (2, 2, 66),
+                                   (3, 4, 9), (2, 5, 70), (2, 8, 33), (3, 13, 64), (2, 16, 37), (2, 17, 130)])
 def test_temporal_carry(dtype, B, T, H):
     from loom_amd import ops
     g = gen(B * T + H)
