@@ -1402,6 +1402,8 @@ final_ca_row_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* _
 namespace loom {
 
 // ---------------------------------------------------------------- dispatch
+constexpr int64_t kTriaPairElements = 1 << 19;
+
 template <typename T, bool PAIR>
 static int tria_depth_launch(const void* r, const void* i, const void* o, const void* prev,
                                const void* seed, const uint8_t* valid, const void* w,
@@ -1441,9 +1443,12 @@ static int tria_depth_dispatch(const void* r, const void* i, const void* o, cons
     // 16-bit element pairs move as one word: H even (a pair stays inside one
     // token) and the element operands 4-byte aligned.  A gated step of 32 x 128 x
     // 3072 in bf16 (529 MB): 93 us, 5.7 TB/s; 104 with one element per thread,
-    // 120 with that and libm's tanh, root and division.
+    // 120 with that and libm's tanh, root and division.  Half a million elements
+    // and fewer are one round of blocks, which half as many only make longer:
+    // steps of 393216 4.95 us against 4.67, of 3072 3.4 against 2.9; of 786432
+    // 6.7 against 8.2.
     if constexpr (sizeof(T) == 2)
-        if (H % 2 == 0 && (((uintptr_t)r | (uintptr_t)i | (uintptr_t)o | (uintptr_t)p_out) & 3) == 0)
+        if (B * T_ * H >= kTriaPairElements && H % 2 == 0 && (((uintptr_t)r | (uintptr_t)i | (uintptr_t)o | (uintptr_t)p_out) & 3) == 0)
             return tria_depth_launch<T, true>(r, i, o, prev, seed, valid, w, carry_out, p_out,
                                               scale_out, B, T_, H, alpha, axis, st);
     return tria_depth_launch<T, false>(r, i, o, prev, seed, valid, w, carry_out, p_out, scale_out, B,

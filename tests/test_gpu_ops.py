@@ -745,11 +745,13 @@ def test_temporal_carry(dtype, B, T, H):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("B,T,H", [(1, 1, 2), (1, 2, 254), (3, 5, 34), (2, 1, 256), (3, 3, 258), (1, 511, 2)])
+@pytest.mark.parametrize("B,T,H", [(1, 1, 2), (1, 2, 254), (3, 5, 34), (2, 1, 256), (3, 3, 258), (1, 511, 2),
+                                   (1, 2048, 256), (2, 2049, 128), (3, 57, 3074), (1, 262145, 2), (5, 53, 2050)])
 @pytest.mark.parametrize("mode", ["init", "seed", "step"])
 def test_tria_depth_element_pairs(dtype, B, T, H, mode):
-    """Two elements per thread (16-bit types, even H, operands aligned to a pair)
-    against one per thread, over whole, ragged and single-pair blocks.  An offset
+    """Two elements per thread (16-bit types, even H, operands aligned to a pair,
+    2^19 elements and more) against one per thread, over whole, ragged and
+    single-pair blocks; the small shapes take one per thread either way.  An offset
     of one element in r takes the call to the form of one element per thread; the
     arithmetic per element is the same, so the results are the same bits."""
     from loom_amd import ops
