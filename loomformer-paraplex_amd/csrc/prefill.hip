@@ -663,19 +663,23 @@ static int prefill_dispatch(const void* qkv, int64_t qkv_ld, void* kc, void* vc,
     const int G = (int)(QH / KVH);
     if constexpr (std::is_same<T, bf16_t>::value) {
         // the MFMA form addresses a (row, kv head)'s cache rows with 32-bit
-        // byte offsets, up to twelve tiles past the chunk's last position
+        // byte offsets, up to four tiles past the chunk's last position (two key
+        // groups: twelve)
+        const auto offsets_fit = [&](int64_t tiles) {
+            return (start + Tc + tiles * kPfRows) * cst * 2 < ((int64_t)1 << 31);
+        };
         const bool mf_ok = (HD == 32 || HD == 64 || HD == 96 || HD == 128) &&
-                           (G == 1 || G == 2 || G == 4 || G == 8) &&
-                           (start + Tc + 12 * kPfRows) * cst * 2 < ((int64_t)1 << 31);
+                           (G == 1 || G == 2 || G == 4 || G == 8) && offsets_fit(4);
         if (mf_ok) {
             // blocks: 4 (query tile, head) pairs each; two key groups per block where a
-            // CU has no more than one block and there are four steps to share (with
-            // RoPE + append, us: 8 x 128 queries over 1152 rows 27.2 -> 23.8, 1 x 128
-            // 25.4 -> 21.7, 16 x 128 over 640 21.4 -> 20.4; 4 x 128 over 138 10.8 -> 11.5).
-            // HD 128's stages fill the LDS with one group.
+            // CU has no more than one block and there are more than four steps to share
+            // (us: 8 x 128 queries over 1152 rows 23.6 -> 19.9, 1 x 128 22.9 -> 19.1, over
+            // 384 10.1 -> 9.6; over 193 and 256 8.2 -> 8.4).  HD 128's stages fill the LDS
+            // with one group.
             const int64_t per = G == 4 ? 16 : G == 8 ? 16 : G == 2 ? 32 : 64;
             const int64_t blocks = ceil_div(Tc, per) * KVH * B * (G == 8 ? 2 : 1);
-            const bool two = HD < 128 && blocks <= (int64_t)device_cus() && start + Tc > 3 * kPfRows;
+            const bool two = HD < 128 && blocks <= (int64_t)device_cus() && start + Tc > 4 * kPfRows &&
+                             offsets_fit(12);
             const dim3 g((unsigned)blocks);
 #define LOOM_PF_GO(HDV, GP, HS)                                                                  \
             do {                                                                                 \
