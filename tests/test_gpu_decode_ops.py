@@ -187,8 +187,8 @@ def test_gqa_prefill_matches_causal_attention(dtype, B, QH, KVH, HD, start, Tc):
 # rows and fewer, 260 blocks and head size 128 keep one group
 @pytest.mark.parametrize("B,QH,KVH,HD,start,Tc", [(1, 8, 2, 96, 0, 129), (2, 8, 2, 96, 0, 200), (1, 8, 8, 64, 77, 130),
                                                   (1, 8, 4, 32, 500, 33), (1, 16, 2, 96, 383, 17), (3, 8, 2, 96, 704, 64),
-                                                  (1, 8, 2, 96, 1500, 1), (65, 8, 2, 32, 100, 32), (1, 8, 2, 128, 250, 50),
-                                                  (2, 8, 2, 96, 0, 300), (1, 8, 8, 64, 127, 130), (3, 8, 2, 96, 239, 17)])
+                                                  (1, 8, 2, 96, 1500, 1), (65, 8, 2, 32, 100, 32), (1, 8, 2, 128, 200, 50),
+                                                  (65, 8, 2, 32, 300, 32), (1, 8, 2, 128, 250, 50), (2, 8, 2, 96, 0, 300), (1, 8, 8, 64, 127, 130), (3, 8, 2, 96, 239, 17)])
 def test_gqa_prefill_two_key_groups(B, QH, KVH, HD, start, Tc):
     test_gqa_prefill_matches_causal_attention(torch.bfloat16, B, QH, KVH, HD, start, Tc)
 
