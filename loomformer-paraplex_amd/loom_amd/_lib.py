@@ -131,7 +131,6 @@ QUERIES = {"loom_gqa_workspace_bytes": ([c_int64] * 5, c_int64),
 
 _lib = None
 _lock = threading.Lock()
-_raw_stream = torch._C._cuda_getCurrentRawStream
 
 DTYPE_CODE = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 
@@ -267,8 +266,10 @@ def addr(t):
 
 
 def raw_stream(device) -> int:
-    """Handle of the current stream of a tensor's device (an int)."""
-    return _raw_stream(device.index)
+    """Handle of the current stream of a tensor's device (an int).  torch's own
+    binding, looked up per call: a torch without a GPU backend has none, and imports
+    this module for its host-only parts."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def ptr(t):

@@ -4,6 +4,8 @@ reference does (no GPU compute here)."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -141,6 +143,18 @@ def test_final_ca_tile_rule():
     for code in (0, 1):
         assert [s for s in faster[code] if not takes(code, *s)] == []
         assert [s for s in slower[code] if takes(code, *s)] == []
+
+
+def test_package_imports_without_a_gpu_build_of_torch():
+    """The host-only parts (configuration, checkpoints, weights, the library's
+    queries) need no GPU backend in torch."""
+    code = ("import sys, torch\n"
+            "if hasattr(torch._C, '_cuda_getCurrentRawStream'): del torch._C._cuda_getCurrentRawStream\n"
+            f"sys.path.insert(0, {os.path.join(ROOT, 'loomformer-paraplex_amd')!r})\n"
+            "from loom_amd import _lib, checkpoint, config, ops, weights\n"
+            "assert _lib.load().loom_abi_version() == 10\n")
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr
 
 
 def test_drop_in_modules_expose_reference_names():
