@@ -137,7 +137,6 @@ def _prefill(eng, prompt: torch.Tensor) -> None:
     trace_p = [[traces[i, bi].data_ptr() for bi in range(L)] for i in (0, 1)]
     kc_p = [t.data_ptr() for t in eng.k_cache]
     vc_p = [t.data_ptr() for t in eng.v_cache]
-    qp_p = [t.data_ptr() for t in eng.qp]
     kvw_p, cos_p, sin_p = eng.kvw.data_ptr(), eng.cos.data_ptr(), eng.sin.data_ptr()
     slot = 2 * N * E                     # bytes of one history slot of a row
     hist_ld = 2 * L * 2 * N              # elements between rows of a history slot
@@ -172,18 +171,11 @@ def _prefill(eng, prompt: torch.Tensor) -> None:
         on main: one pass over slots [0, sub] for sublayers sub and sub + 1 (the
         latter's part over them in fp32), then the fold of the last slot."""
         if not pair:
-            if eng.depth_rms is None:
-                call("loom_depth_attn_forward", code, qp_p[sub], hist_p, hist_p + N * E, hist_ld, 2 * N, out_p, None,
-                     None, rows, sub + 1, QH, HD, st)
-            else:
-                call("loom_depth_attn_forward_rms", code, qp_p[sub], hist_p, hist_p + N * E, hist_ld, 2 * N, out_p,
-                     None, None, rows, sub + 1, QH, HD, *eng.depth_rms, st)
+            eng._depth_read(sub, hist_p, out_p, rows, st)
         elif sub % 2 == 0:
-            call("loom_depth_attn_pair", code, qp_p[sub], qp_p[sub + 1], hist_p, hist_p + N * E, hist_ld, 2 * N,
-                 out_p, part_d_p, part_lse_p, rows, sub + 1, QH, HD, st)
+            eng._depth_read_pair(sub, hist_p, out_p, part_d_p, part_lse_p, rows, st)
         else:
-            call("loom_depth_attn_fold", code, qp_p[sub], hist_p, hist_p + N * E, hist_ld, 2 * N, sub + 1, part_d_p,
-                 part_lse_p, out_p, rows, QH, HD, st)
+            eng._depth_read_fold(sub, hist_p, out_p, part_d_p, part_lse_p, rows, st)
 
     spans = list(zip([0] + [x + 1 for x in ends[:-1]], ends))
 
