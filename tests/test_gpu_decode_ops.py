@@ -265,12 +265,26 @@ def test_staged_tiles_with_ragged_rows(M, shared):
     """The DMA-staged tiles store a last row tile with rows missing as they
     store a whole one (row-masked): plain, gated + residual, split-K +
     LayerNorm and RoPE epilogues; nothing is written past row M."""
+    _ragged_rows_case(M, 768, 768, shared)
+
+
+@pytest.mark.parametrize("M,N,K", [(8191, 512, 2048), (8192, 512, 2048), (2001, 2048, 512), (4097, 512, 512)])
+def test_staged_128_tiles_with_ragged_rows(M, N, K):
+    """The same of the 128 x 128 tiles (K a multiple of 128 but not of 192)."""
+    f = L().load().loom_test_gemm_kernel
+    f.argtypes = [ctypes.c_int] + [ctypes.c_int64] * 4 + [ctypes.c_int]
+    assert f(1, M, N, K, 0, 1) == 2 and (M < 5000 or f(1, M, N, K, 0, 0) == 2)
+    _ragged_rows_case(M, N, K, False)
+
+
+def _ragged_rows_case(M, N, K, shared):
     from loom_amd import _lib, ops
-    bf, K, N = torch.bfloat16, 768, 768
+    bf = torch.bfloat16
     g = torch.Generator().manual_seed(M)
     r = lambda *s, sc=1.0: (torch.randn(*s, generator=g) * sc).to(DEV, bf)
     x, w, p, res = r(M, K), r(N, K, sc=K ** -0.5), r(M, N), r(M, N)
     bias, gam, bet = (torch.randn(N, generator=g).to(DEV) for _ in range(3))
+    w2 = w if N == K else r(N, N, sc=N ** -0.5)
     want = host(x) @ host(w).T
     nb = _lib.load().loom_linear_ln_workspace_bytes(M, N)
     ws = torch.empty(nb // 4, device=DEV)
@@ -282,12 +296,12 @@ def test_staged_tiles_with_ragged_rows(M, shared):
             check(out[:M], ref_ + host(bias), bf)
             assert bool((out[M:] == 7.0).all())
         y, out = torch.zeros(M, N, device=DEV, dtype=bf), torch.full((M + 3, N), 7.0, device=DEV, dtype=bf)
-        d = _lib.linear_multi_desc(x, [dict(w=w, w2=w, out=y, bias=bias)], x2=p)
+        d = _lib.linear_multi_desc(x, [dict(w=w, w2=w2, out=y, bias=bias)], x2=p)
         _lib.call("loom_linear_ln", code(x), ctypes.byref(d), P(gam), P(bet), 1e-5, P(out), N, P(ws), nb, None, S(x))
-        check(out[:M], torch.nn.functional.layer_norm(want + host(p) @ host(w).T + host(bias), (N,), host(gam),
+        check(out[:M], torch.nn.functional.layer_norm(want + host(p) @ host(w2).T + host(bias), (N,), host(gam),
                                                       host(bet), 1e-5), bf)
         assert bool((out[M:] == 7.0).all())
-    if M == 3131:
+    if M == 3131 and K == 768:
         with shared_tiles(shared):
             _prefill_qkv_case(bf, 31, 101, 5, 96, True)
 
@@ -304,12 +318,13 @@ def shared_tiles(on):
 
 
 @pytest.mark.parametrize("M,N,K", [(4096, 3072, 768), (4000, 1152, 768), (300, 768, 1536),
-                                   (4096, 768, 3072), (4096, 1536, 768)])
+                                   (4096, 768, 3072), (4096, 1536, 768), (3001, 768, 1536)])
 def test_shared_tiles_equal_default_tiles(M, N, K):
     """Shared-tile mode (128 x 192 tiles of four waves, two blocks per CU)
     against the default tiles: loom_linear with bias, gate and residual and
     loom_linear_ln (whose split-K count may differ) against torch in both
-    modes, the W_imag gather product of both modes against each other."""
+    modes, the W_imag gather product of both modes against each other.  (300 rows
+    take the direct fragments in both modes.)"""
     from loom_amd import _lib, ops
     dt = torch.bfloat16
     g = torch.Generator().manual_seed(M + N + K)
@@ -866,7 +881,9 @@ def test_ffn_decode_with_depth_read(dtype, M, rms, slots, QH, HD, part):
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("M,K2,N", [(1, 768, 768), (4, 3072, 768), (32, 768, 768), (32, 3072, 768),
                                     (64, 3072, 768), (7, 0, 768), (4096, 768, 768), (4096, 3072, 768),
-                                    (300, 768, 768), (512, 0, 768), (520, 768, 200)])
+                                    (300, 768, 768), (512, 0, 768), (520, 768, 200),
+                                    # direct fragments over both inputs, 64 x 32 and 64 x 64 tiles
+                                    (512, 768, 768), (777, 768, 768), (999, 3072, 768)])
 def test_linear_ln(dtype, M, K2, N):
     """LayerNorm(x w^T + x2 w2^T + b): split-K partial sums reduced inside the
     LayerNorm kernel (bf16: the skinny form up to 64 rows, the 256 x 128 MFMA
