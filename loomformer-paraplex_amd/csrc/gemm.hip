@@ -1673,8 +1673,19 @@ static void launch_frag_cfg(const GemmArgs& a, hipStream_t st) {
     const dim3 grid((unsigned)(ceil_div(a.M, C::TM) * ceil_div(a.N, C::TN)));
     hipLaunchKernelGGL((gemm_frag_kernel<T, MT, NT, KW, U, GATHER, DUAL>), grid, dim3(C::THREADS), 0, st, a);
 }
+// k parts (waves of a block) and units in flight of each tile.  64 x 32: eight parts
+// in bf16 and four in fp32, whose waves the matrix cores bound (512 x 768 x 3072 14.3
+// us with eight against 14.8 with four in bf16, 37.6 against 36.0 in fp32); a second
+// unit in flight is slower there (500 x 768 x 768 5.8 -> 6.2, fp32 11.6 -> 11.9).
+// The smaller tiles' counts were set while the launch gaps hid the difference: as
+// captured launches with operands in the L2, four parts and one unit take 3.2 us
+// where 16 x 16 tiles of sixteen take 3.7 (33 x 768 x 768; 64 x 768 x 3072 6.3, 6.6),
+// 32 x 16 tiles in bf16 3.7 against 4.3 (32 x 3072 x 768; fp32 has eight parts and
+// one unit first, 5.5 against 6.3), 32 x 32 tiles 4.2 against 4.7 (64 x 3072 x 768).
+
 // k parts of the 64 x 64 tiles: eight (one block per CU) or four (two blocks per
-// CU), whichever fills its rounds better
+// CU), whichever fills its rounds better (333 x 3072 x 768, 288 tiles: 13.3 us with
+// eight, 11.2 with four; 999 x 768 x 3072, 192 tiles: 20.2 and 20.7)
 static int frag_wide_parts(int64_t M, int64_t N) {
     const int64_t n = ceil_div(M, 64) * ceil_div(N, 64), c = device_cus();
     return n <= c || ceil_div(n, c) < 2 * ceil_div(n, 2 * c) ? 8 : 4;
