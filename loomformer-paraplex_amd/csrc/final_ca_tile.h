@@ -1,7 +1,8 @@
 // Sequence form of the sparse final cross-attention on the matrix cores
 // (included by tria.hip): 16 query rows of one batch row per block, so the
 // block's keys and values are read once for 16 rows (the one-row kernels read
-// them once per row: 8 x 2048 rows over 15 keys of 768 in bf16 253 us).
+// them once per row: 8 x 2048 rows over 15 keys of 768 in bf16 253 us, here 14; on
+// operands no cache holds yet, launch included, 283 and 38).
 //
 // Four waves share the D dimensions in slabs of 64: wave w takes slabs w, w+4,
 // ... of the scores S = K Q^T (summed over the waves through LDS) and then of

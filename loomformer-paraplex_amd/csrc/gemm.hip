@@ -1569,9 +1569,9 @@ static void launch_skinny(const GemmArgs& a, dim3 grid, hipStream_t st) {
 //   256 x 128 otherwise, and 128 x 128 only where 256 x 128 cannot run (fewer
 //     than 256 rows, K not a whole round of its stages).  Alone, 128 x 128 is
 //     faster whenever 256 x 128 leaves CUs idle (4096 x 768 x 3072: 32.5
-//     against 47.0 us), but inside the chunked prefill, beside the other
-//     streams' kernels, choosing it there measured 74.4-75.2 ms against
-//     73.5-74.0 ms (same box, alternating runs).
+//     against 47.0 us); the order is from when the chunked prefill ran on these
+//     tiles, where it measured slower beside the other streams' kernels (74.4-75.2
+//     ms against 73.5-74.0).  The prefill takes 128 x 192 in shared-tile mode now.
 // K must fill whole rounds of the configuration's stages; gather tiles must
 // not straddle a q-head group (Hq % BG_N == 0).
 enum BigTile { kBigNone, kBigStd, kBigSmall, kBigWide, kBigTall, kBigTallS };
