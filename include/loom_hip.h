@@ -495,8 +495,8 @@ int loom_gemm_shared_tiles(int on);
  * and strides as there), and, with w_hist set, the depth history slot's
  * projection hist_out = x w_hist^T (DepthAttn.project, loomformer.py:3397;
  * n_hist columns at hist_ld elements apart).  Weights are [rows, K] dense.
- * Follow it with loom_gqa_prefill(qkv = NULL).  bf16 with head_dim 96 and at
- * least 256 rows runs as one launch that never stores qkv; other shapes use
+ * Follow it with loom_gqa_prefill(qkv = NULL).  bf16 with head_dim 96 and
+ * many rows runs as one launch that never stores qkv; other shapes use
  * qkv_scratch ([B*T, (QH + 2 KVH) HD]) and a separate RoPE + append launch.
  * No counterpart in the reference. */
 int loom_prefill_qkv(int dtype, const void* x, int64_t ldx, const void* w_qkv, const void* w_hist,

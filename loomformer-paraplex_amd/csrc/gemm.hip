@@ -1720,14 +1720,12 @@ static int64_t staged_ns(BigTile tile, int64_t M, int64_t N, int64_t K, bool gat
     return ceil_div(blocks, per_cu * (int64_t)device_cus()) * (fixed + K * per10 / 10);
 }
 
-// A direct-fragment product's time for this comparison: frag_tile's, and more for
-// further rounds, two of which run as one of two blocks per CU (measured, estimated
-// us: two rounds 1024 x 1152 x 768 12.6, 11.9; three 999 x 3072 x 1152 of the gather
-// 26.5, 24.4, 1280 x 2048 x 768 of it 19.7, 18.3)
+// A direct-fragment product's time for this comparison: frag_tile's, and 1500 ns
+// for each further round (999 x 3072 x 1152 of the gather 26.5 us, three rounds of
+// 5.9 and 3; two rounds 2500 x 768 x 768 13.4, 1024 x 1152 x 768 12.5 as staged)
 static int64_t frag_ns(const GemmArgs& a, bool gather) {
     const FragTile t = frag_tile<bf16_t>(a.M, a.N, a.K, gather, a.Hq);
-    const int64_t rounds = ceil_div(ceil_div(a.M, t.tm) * ceil_div(a.N, t.tn), (int64_t)device_cus());
-    return t.ns + (rounds <= 2 ? 700 : 1500) * (rounds - 1);
+    return t.ns + 1500 * (ceil_div(ceil_div(a.M, t.tm) * ceil_div(a.N, t.tn), (int64_t)device_cus()) - 1);
 }
 
 // bf16: the direct-fragment kernels or the DMA-staged tiles.  Over 14 widths of 512
@@ -2516,8 +2514,8 @@ extern "C" int loom_beta_forward(int dtype, const void* u, const void* q_h, cons
 // The chunked prefill's projections of one hidden state for the next block:
 // qkv = x w_qkv^T, then RoPE of q and k and the cache append of k and v
 // (as loom_gqa_prefill's first step), and optionally the history projection
-// hist_out = x w_hist^T.  bf16 with 96-wide heads and at least 256 rows: one
-// launch of 256 x 192 tiles, the RoPE and the cache stores in its epilogue
+// hist_out = x w_hist^T.  bf16 with 96-wide heads and many rows (where it is the
+// faster way): one launch of 256 x 192 tiles, the RoPE and the cache stores in its epilogue
 // (each wave's 96 columns are one head) and the history columns as a second
 // product of the same launch; qkv is never stored.  Otherwise the two
 // products into qkv_scratch / hist_out and the separate RoPE + append launch.
@@ -2525,13 +2523,15 @@ extern "C" int loom_gemm_shared_tiles(int on) {
     return g_shared_tiles.exchange(on != 0 ? 1 : 0);
 }
 
-// One launch, or the products by themselves and the RoPE launch: the staged tiles'
-// estimate with the RoPE epilogue's registers to move (256 x 192 tiles 15000 ns more,
-// 128 x 192 6500), against the products' and 3000 ns + 1 ns per 900 elements
-// of q, k and v (read and written; rows of 1152 + 1536 columns of 768, 128 x 192 tiles: 512 rows
-// 19.2 us against 17.7, 768 20.3 and 22.1, 1024 21.4 and 26.5; without the history
-// columns 512 18.7 and 10.5, 1536 19.8 and 16.4, 2048 19.4 and 24.9)
+// One launch, or the products by themselves and the RoPE launch.  The result is that
+// of loom_linear to the bit, so where loom_linear takes the direct fragments qkv
+// does too.  Else by the staged tiles' estimate with the RoPE epilogue's registers to
+// move (256 x 192 tiles 15000 ns more, 128 x 192 6500) against the products' and
+// 3000 ns + 1 ns per 900 elements of q, k and v (rows of 1152 + 1536 columns of 768
+// in 128 x 192 tiles against separate: 1024 rows 21.4 us and 26.5, 1792 22.3 and 36;
+// 1536 rows without the history columns 19.8 and 17.5)
 static bool prefill_qkv_fused_faster(const GemmArgs& qkv, const void* w_hist, int64_t n_hist, bool shared) {
+    if (frag_fits<bf16_t, false>(qkv) && takes_frag(qkv, false, big_tile(qkv.M, qkv.N, qkv.K, false, 0), false)) return false;
     GemmArgs h = qkv;
     h.W = w_hist;
     h.N = n_hist;

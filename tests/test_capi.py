@@ -111,7 +111,7 @@ def test_product_kernel_rule():
     for M in (768, 777, 1024):
         assert of(M, 3072, 1152, hd=96, shared=1) == 5
     # and slower
-    for s in [(999, 768, 3072), (512, 768, 768), (1024, 768, 768), (512, 3072, 768), (1024, 512, 2048), (512, 1024, 1024)]:
+    for s in [(999, 768, 3072), (512, 768, 768), (1024, 768, 768), (300, 3072, 768), (1024, 512, 2048), (512, 1024, 1024)]:
         assert of(*s) > 100, s
     assert of(600, 4096, 1536, hd=128) > 100 and of(333, 3072, 1152, hd=96, shared=1) > 100
     # few rows: the skinny kernel up to 24 rows of few k
@@ -121,7 +121,7 @@ def test_product_kernel_rule():
     for M in (384, 512, 768, 1024):
         for N in (3072, 1536, 4608):
             assert of(M, N, 768, multi=1) in (1, 2, 3, 4)
-    assert of(300, 4608, 768, multi=1) > 100 and of(256, 6144, 1024, multi=1) < 100
+    assert of(300, 3072, 768, multi=1) > 100 and of(256, 6144, 1024, multi=1) < 100
 
 
 def test_final_ca_tile_rule():

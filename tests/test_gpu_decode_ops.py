@@ -198,10 +198,16 @@ def test_gqa_prefill_two_key_groups(B, QH, KVH, HD, start, Tc):
                                                        (16, 17, 500, 96, False, False),
                                                        (2, 20, 3, 96, True, False), (4, 70, 9, 64, True, False),
                                                        (32, 128, 37, 96, True, True),
-                                                       (16, 17, 500, 96, False, True)])
+                                                       (16, 17, 500, 96, False, True),
+                                                       # around the lines between one launch, the staged
+                                                       # products and the direct fragments
+                                                       (6, 128, 5, 96, True, True), (8, 97, 0, 96, True, True),
+                                                       (8, 128, 0, 96, True, True), (12, 128, 0, 96, True, True),
+                                                       (13, 120, 7, 96, False, True), (20, 128, 0, 96, False, True),
+                                                       (8, 128, 0, 96, True, False), (12, 127, 0, 96, False, False)])
 def test_prefill_qkv_matches_products_and_rope(dtype, B, Tc, start, HD, hist, shared):
     """loom_prefill_qkv = the qkv product, loom_gqa_prefill's RoPE + cache append
-    and the history projection, to the bit (bf16, head_dim 96, >= 256 rows: one
+    and the history projection, to the bit (bf16, head_dim 96, many rows: one
     launch with the RoPE in the product's epilogue; the rest: the separate
     products and RoPE launch), and against torch: the product rounded to the
     dtype, then the oracle's RoPE.  `shared`: in shared-tile mode (128 x 192

@@ -258,7 +258,7 @@ def product_kernel(dtype, *args):
     (17, 64, 64, 0, 1616), (25, 64, 64, 1616, 1616), (33, 40, 192, 1616, 1616), (47, 1000, 768, 1616, 1616),
     (31, 3072, 768, 3216, 3216), (130, 768, 3072, 3216, 3216), (64, 3072, 768, 3232, 3232),
     (65, 768, 1536, 1616, 1616), (129, 1500, 768, 3232, 3232), (255, 768, 3072, 3232, 3232),
-    (500, 770, 768, 6432, 6432), (513, 3072, 320, 46464, 46464), (1100, 1500, 768, 46464, 46464),
+    (500, 770, 768, 6432, 6432), (513, 3072, 320, 46464, 46464), (1100, 1500, 768, 1, 46464),
     (999, 768, 3072, 86464, 86464), (1000, 3100, 768, 1, 46464), (2100, 4000, 64, 86464, 86464)])
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_direct_fragment_products(dtype, M, N, K, k16, k32):
