@@ -131,6 +131,9 @@ QUERIES = {"loom_gqa_workspace_bytes": ([c_int64] * 5, c_int64),
 
 _lib = None
 _lock = threading.Lock()
+# (a torch without a GPU backend has no such binding and no device tensors either;
+# it imports this module for its host-only parts)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 DTYPE_CODE = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 
@@ -266,10 +269,8 @@ def addr(t):
 
 
 def raw_stream(device) -> int:
-    """Handle of the current stream of a tensor's device (an int).  torch's own
-    binding, looked up per call: a torch without a GPU backend has none, and imports
-    this module for its host-only parts."""
-    return torch._C._cuda_getCurrentRawStream(device.index)
+    """Handle of the current stream of a tensor's device (an int)."""
+    return _raw_stream(device.index)
 
 
 def ptr(t):
